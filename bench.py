@@ -568,10 +568,10 @@ def main() -> int:
     salu_peak = cus * CLOCK_GHZ  # G SALU instructions/s
     salu_achieved = ISSUE_COUNTS["salu"] / max(1, launches) / per_launch_s / 1e9
     # Beside it: the LDS bytes the stash moves (each promise that passes
-    # through it is written into a link and read back out, 2 x 16 B; promises
-    # run by link forwarding stay in registers) against 128 B per CU per
-    # clock, and the measured HBM traffic against the HBM peak.
-    stashed = promises - runs[-1]["forwarded"]
+    # through it is written into a link and read back out, 2 x 16 B; where
+    # lanes chain that is one promise per start at most) against 128 B per CU
+    # per clock, and the measured HBM traffic against the HBM peak.
+    stashed = COUNT
     lds_achieved = 2 * PROMISE_BYTES * stashed / max(1, launches) / per_launch_s / 1e9
     lds_peak = cus * LDS_BYTES_PER_CLOCK_PER_CU * CLOCK_GHZ
     hbm_achieved = measured_traffic_bytes() / per_launch_s / 1e9
@@ -618,8 +618,8 @@ def main() -> int:
             "counts_per_launch": {k: v / max(1, launches) for k, v in ISSUE_COUNTS.items()},
             "counters": "profiles/collatz_async_issue_counters.md",
             "lds": {"achieved": lds_achieved, "peak": lds_peak, "unit": "GB/s", "frac": lds_achieved / lds_peak,
-                    "rule": "2 x 16 B per promise through the stash (write + read; forwarded promises skip "
-                            "it); peak 128 B per CU per clock"},
+                    "rule": "2 x 16 B per promise through the stash (write + read; at most one per start, the "
+                            "others stay in registers); peak 128 B per CU per clock"},
             "hbm": {"achieved": hbm_achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                     "frac": hbm_achieved / HBM_PEAK_GBPS, "rule": "measured traffic per launch / launch time"},
             "algorithmic_hbm_equivalent": {

@@ -353,28 +353,27 @@ class AsyncProgram {
     static_assert(LAZY_WORDS <= 16, "a LazyLoad value may span at most 16 words");
     static constexpr uint32_t SPARES = 4;
 
-    // Link forwarding. While a link is evaluated, each lane's first async
-    // call (at the caller's depth level) is held in the lane's registers
-    // instead of being appended to the stash. If afterwards every held
-    // promise names the same operation and at least FORWARD_MIN lanes hold
-    // one, those promises run at once as a link of their own, straight from
-    // registers, and so on for up to FORWARD_RUNS links; otherwise, and
-    // after the last forwarded run, the held promises are appended to the
-    // stash as usual. A full link of one operation whose promises each queue
-    // one promise of another (a Collatz odd step is always followed by an
-    // even one) thus skips the stash's append, bookkeeping and read for its
-    // successor link (Collatz 2^26: 58.9 -> 52.1 ms per launch). Order of
-    // evaluation is all that changes. Only flat programs (one depth level)
-    // without asynchronous argument loads forward, and a specification can
-    // turn it off (FORWARD_LINKS = 0).
-#ifndef HZ_FORWARD
-#define HZ_FORWARD 1
+    // Lane chaining. While promises are evaluated, each lane's first async
+    // call stays in the lane's registers and is the promise the lane runs
+    // next. Lanes whose chain has ended are filled again from the stash, and
+    // only further calls of a lane (a split, a fan-out) are appended to it,
+    // so a chain of single successors passes through LDS once, at its start,
+    // instead of once per promise. Order of evaluation is all that changes.
+    // Only flat programs (one depth level) without asynchronous argument
+    // loads chain, and a specification can turn it off (CHAIN_LANES = 0, or
+    // FORWARD_LINKS = 0 without CHAIN_LANES).
+    //
+    // CHAIN_MIN: lanes that must hold a promise for the next pass to run
+    // without looking for more work. CHAIN_RUNS: evaluations between two
+    // visits to the scheduler (spills, flags, queues).
+#ifndef HZ_CHAIN
+#define HZ_CHAIN 1
 #endif
-#ifndef HZ_FORWARD_MIN
-#define HZ_FORWARD_MIN 48
+#ifndef HZ_CHAIN_MIN
+#define HZ_CHAIN_MIN 60
 #endif
-#ifndef HZ_FORWARD_RUNS
-#define HZ_FORWARD_RUNS 4
+#ifndef HZ_CHAIN_RUNS
+#define HZ_CHAIN_RUNS 512
 #endif
     // Layout of a link's promise words, the same in the stash and in the
     // arena (so moving a link is a flat copy): promise-major when a promise
@@ -388,10 +387,29 @@ class AsyncProgram {
         return PROMISE_MAJOR ? promise * WORDS + word : word * 64u + promise;
     }
 
-    static constexpr bool FORWARD = HZ_FORWARD != 0 && hz::spec::FORWARD_LINKSOr<PROGRAM_SPEC, 1>::value != 0 &&
-                                    LEVELS == 1 && !HAS_LAZY;
-    static constexpr uint32_t FORWARD_MIN = HZ_FORWARD_MIN;
-    static constexpr uint32_t FORWARD_RUNS = HZ_FORWARD_RUNS;
+    static constexpr bool FORWARD = hz::spec::FORWARD_LINKSOr<PROGRAM_SPEC, 1>::value != 0;
+    static constexpr bool CHAIN = HZ_CHAIN != 0 && LEVELS == 1 && !HAS_LAZY && OPS > 0 &&
+                                  hz::spec::CHAIN_LANESOr<PROGRAM_SPEC, FORWARD ? 1 : 0>::value != 0;
+    static constexpr uint32_t CHAIN_MIN = HZ_CHAIN_MIN;
+    // (A program that shares work consults its hungry count between them.)
+    static constexpr uint32_t CHAIN_RUNS = SHARE_WORK ? 8u : (uint32_t)HZ_CHAIN_RUNS;
+    // Lanes holding different operations run one operation after another in
+    // one pass. With up to two operations every pass is at least half full,
+    // which costs less than a trip through the stash; with more, the lanes
+    // of the most common operation go on and the others return to the stash,
+    // which coalesces them.
+    static constexpr bool CHAIN_MIXED = hz::spec::CHAIN_MIXEDOr<PROGRAM_SPEC, OPS <= 2 ? 1 : 0>::value != 0;
+    // One operation's promises are never queued and run in the same pass.
+    static constexpr bool COUNT_FORWARDED = CHAIN && FORWARD && OPS > 1;
+    // Passes run between two looks at how many lanes still hold a promise.
+    static constexpr uint32_t CHAIN_PASSES = (uint32_t)hz::spec::CHAIN_PASSESOr<PROGRAM_SPEC, 1>::value;
+    static_assert(CHAIN_PASSES >= 1 && CHAIN_PASSES <= 16, "CHAIN_PASSES must be in [1, 16]");
+    // Evaluations without a refill after which lanes that go on chaining
+    // make room for what waits in the stash, so that promises that requeue
+    // themselves until another promise has run cannot keep it waiting.
+    static constexpr uint32_t CHAIN_TURN = 1024;
+    // A launch's cycle budget counts evaluations in units of this many.
+    static constexpr uint32_t RUNS_PER_CYCLE = 8;
 
     static const unsigned int BAD_FUNC_ID_FLAG = 0x00000001;
     static const unsigned int STASH_FAIL_FLAG = 0x00000002;
@@ -420,9 +438,10 @@ class AsyncProgram {
     struct ThreadContext {
         unsigned int thread_id;
         unsigned int rand_state;
-        // Promises this lane wrote into links. Counted per lane, in a
-        // register: appends run in divergent code, where a shared counter
-        // would need a cross-lane ordering on every call.
+        // Promises this lane's async calls wrote into links. Counted per
+        // lane, in a register: appends run in divergent code, where a shared
+        // counter would need a cross-lane ordering on every call. (Promises
+        // held by lane chaining are counted in `held`.)
         unsigned long long appended;
         // Promises evaluated and links run by this lane's group: the same
         // value in every lane, kept in registers rather than read and
@@ -436,13 +455,27 @@ class AsyncProgram {
         uint32_t idle_streak;      // consecutive idle cycles
         uint32_t queue_check;      // cycles until the device queues are consulted again
         uint32_t make_pause;       // cycles before make_work is called again (pause_make_work)
-        // Link forwarding: whether async calls are held (uniform; set while
-        // a link is evaluated), and this lane's held promise (its operation,
-        // LINK_NONE if none, and its words).
-        uint32_t fwd_on;
-        uint32_t fwd_op;
-        uint32_t fwd_words[FORWARD ? WORDS : 1];
-        unsigned long long forwarded;  // promises the group ran by forwarding (uniform)
+        uint32_t queue_pause;      // CHAIN: cycles added to queue_check by the last check that found nothing
+        uint32_t cycle_runs;       // links evaluated in the current cycle
+        // Lane chaining: whether async calls are held (uniform; set while
+        // promises are evaluated or made), and the promise this lane runs
+        // next (its operation, LINK_NONE if none, and its words).
+        uint32_t chain_on;
+        uint32_t chain_op;
+        uint32_t chain_words[CHAIN ? WORDS : 1];
+        // The stash link that lanes are being filled from (LINK_NONE if
+        // none), out of the stash's own tables, its operation and the
+        // promises left in it (uniform).
+        uint32_t feed_link;
+        uint32_t feed_op;
+        uint32_t feed_count;
+        uint32_t chain_streak;         // evaluations since a link was last taken to fill lanes (uniform)
+        uint32_t chain_turn;           // stash link the last turn ran (uniform)
+        unsigned long long chained;    // promises this lane ran chaining
+        // With the `chained` counts, the promises the group's lanes have held
+        // (uniform; wraps below zero).
+        unsigned long long held;
+        unsigned long long forwarded;  // promises this lane ran in the pass that queued them
     };
 
     // Per-wavefront scheduler state, in LDS.
@@ -977,7 +1010,6 @@ class AsyncProgram {
         const uint32_t slot = D * LEVELS + lv;
         const uint32_t entry = hz::wave::first(g.open[slot]);
         uint32_t L, c = 0;
-        _thd_ctx.appended += 1u;
         if (entry == hz::LINK_NONE) {
             L = take_link();
             if (L == hz::LINK_NONE) return;
@@ -1056,14 +1088,15 @@ class AsyncProgram {
         pu.template cast<TYPE>() = param_value;
         uint32_t words[WORDS];
         __builtin_memcpy(words, &pu, sizeof(PromiseUnionType));
-        if constexpr (FORWARD) {
-            if (depth_delta == 0 && hz::wave::first(_thd_ctx.fwd_on) != 0u && _thd_ctx.fwd_op == hz::LINK_NONE) {
-                _thd_ctx.fwd_op = D;
+        if constexpr (CHAIN) {
+            if (hz::wave::first(_thd_ctx.chain_on) != 0u && _thd_ctx.chain_op == hz::LINK_NONE) {
+                _thd_ctx.chain_op = D;
 #pragma unroll
-                for (uint32_t w = 0; w < WORDS; ++w) _thd_ctx.fwd_words[w] = words[w];
+                for (uint32_t w = 0; w < WORDS; ++w) _thd_ctx.chain_words[w] = words[w];
                 return;
             }
         }
+        _thd_ctx.appended += 1u;
         stash_append(D, child_level(depth_delta), words);
     }
 
@@ -1141,9 +1174,15 @@ class AsyncProgram {
 
     __device__ bool stash_empty() { return hz::wave::first(_grp_ctx.free_mask) == ALL_LINKS; }
 
+    // Lanes that hold a promise to run next (CHAIN; every lane active).
+    __device__ HZ_INLINE uint64_t held_lanes() {
+        if constexpr (!CHAIN) return 0ull;
+        return hz::wave::ballot(_thd_ctx.chain_op != hz::LINK_NONE);
+    }
+
     __device__ HZ_INLINE void drop_holding_if_empty() {
         GroupContext& g = _grp_ctx;
-        if (stash_empty() && hz::wave::first(g.holding)) {
+        if (stash_empty() && held_lanes() == 0ull && hz::wave::first(g.holding)) {
             if (hz::wave::lane() == 0) {
                 g.holding = 0;
                 add_units(-1);
@@ -1162,10 +1201,16 @@ class AsyncProgram {
         const uint32_t lane = hz::wave::lane();
         _thd_ctx.made += 1u;
         if constexpr (LEVELS > 1) g.level = 0u;
+        // A lane without a promise keeps the first one it makes.
+        const uint64_t before = held_lanes();
+        _thd_ctx.chain_on = CHAIN && CHAIN_MIXED ? 1u : 0u;
         bool mine;
         [[clang::always_inline]] mine = PROGRAM_SPEC::make_work(*this);
+        _thd_ctx.chain_on = 0u;
         bool more = hz::wave::ballot(mine) != 0;
-        const bool holds = !stash_empty();
+        const uint64_t now = held_lanes();
+        _thd_ctx.held += hz::wave::popc(now & ~before);
+        const bool holds = now != 0ull || !stash_empty();
         if (lane == 0) {
             if (holds && !g.holding) {
                 g.holding = 1;
@@ -1294,7 +1339,6 @@ class AsyncProgram {
         }
         {
             HZ_PHASE(PHASE_EVAL);
-            if constexpr (FORWARD) _thd_ctx.fwd_on = 1u;
             if (lane < cnt) {
                 PromiseUnionType pu;
                 __builtin_memcpy(&pu, words, sizeof(PromiseUnionType));
@@ -1304,52 +1348,334 @@ class AsyncProgram {
                 pu.template loose_eval<ProgramType>(*this, op);
             }
             hz::wave::sync();
-            if constexpr (FORWARD) run_forwarded();
         }
     }
 
-    // Runs the promises the lanes hold in registers while they form a link
-    // of one operation of at least FORWARD_MIN lanes (at most FORWARD_RUNS
-    // such links), then appends what is still held to the stash.
-    __device__ HZ_INLINE void run_forwarded() {
-        for (uint32_t k = 0; k < FORWARD_RUNS; ++k) {
-            const uint64_t held = hz::wave::ballot(_thd_ctx.fwd_op != hz::LINK_NONE);
-            if (held == 0ull) break;
-            const uint32_t D = hz::wave::read_lane(_thd_ctx.fwd_op, (uint32_t)__builtin_ctzll(held));
-            const uint64_t same = hz::wave::ballot(_thd_ctx.fwd_op == D);
-            const uint32_t n = (uint32_t)__builtin_popcountll(same);
-            if (same != held || n < FORWARD_MIN) break;
-            uint32_t words[WORDS];
+    // ---------------------------------------------------------- lane chaining
+    // Takes stash link L as the one that lanes are filled from.
+    __device__ HZ_INLINE void take_feed(uint32_t L) {
+        GroupContext& g = _grp_ctx;
+        const uint32_t rm = hz::wave::first(g.ready_mask);
+        _thd_ctx.feed_link = L;
+        _thd_ctx.feed_op = hz::wave::first(g.link_op[L]);
+        _thd_ctx.feed_count = hz::wave::first(g.link_count[L]);
+        if (((rm >> L) & 1u) != 0u) {
+            g.ready_mask = rm & ~(1u << L);
+        } else {
+            g.open[open_index(L)] = hz::LINK_NONE;
+        }
+        hz::wave::sync();
+    }
+
+    // Hands what is left of the feed back to the stash, as a ready link.
+    __device__ HZ_INLINE void return_feed() {
+        GroupContext& g = _grp_ctx;
+        if (hz::wave::first(_thd_ctx.feed_link) == hz::LINK_NONE) return;
+        const uint32_t L = hz::wave::first(_thd_ctx.feed_link);
+        g.link_count[L] = _thd_ctx.feed_count;
+        g.ready_mask = hz::wave::first(g.ready_mask) | (1u << L);
+        _thd_ctx.feed_link = hz::LINK_NONE;
+        _thd_ctx.feed_count = 0u;
+        hz::wave::sync();
+    }
+
+    // Fills lanes without a promise from the feed (every lane active; `held`
+    // lanes have one), its last promises first; returns the lanes that hold
+    // one afterwards. The feed's state is in registers, so this costs one LDS
+    // access per lane filled and no round trip for bookkeeping.
+    __device__ HZ_INLINE uint64_t fill_lanes(uint64_t held) {
+        GroupContext& g = _grp_ctx;
+        const uint64_t idle = ~held;
+        const uint32_t L = hz::wave::first(_thd_ctx.feed_link);
+        const uint32_t cnt = hz::wave::first(_thd_ctx.feed_count);
+        const uint32_t want = hz::wave::popc(idle);
+        const uint32_t k = want < cnt ? want : cnt;
+        const uint32_t r = hz::wave::rank(idle);
+        if (_thd_ctx.chain_op == hz::LINK_NONE && r < k) {
 #pragma unroll
-            for (uint32_t w = 0; w < WORDS; ++w) words[w] = _thd_ctx.fwd_words[w];
-            const bool mine = _thd_ctx.fwd_op != hz::LINK_NONE;
-            _thd_ctx.fwd_op = hz::LINK_NONE;
-            _thd_ctx.executed += n;
-            _thd_ctx.runs += 1u;
-            _thd_ctx.forwarded += n;
-            if (mine) {
-                _thd_ctx.appended += 1u;  // counted as written into a link, as an append would
-                PromiseUnionType pu;
-                __builtin_memcpy(&pu, words, sizeof(PromiseUnionType));
-                pu.template loose_eval<ProgramType>(*this, D);
-            }
+            for (uint32_t w = 0; w < WORDS; ++w) _thd_ctx.chain_words[w] = g.words[L][word_index(cnt - k + r, w)];
+            _thd_ctx.chain_op = _thd_ctx.feed_op;
+        }
+        hz::wave::sync();
+        _thd_ctx.feed_count = cnt - k;
+        if (k == cnt) {
+            g.free_mask = hz::wave::first(g.free_mask) | (1u << L);
+            _thd_ctx.feed_link = hz::LINK_NONE;
             hz::wave::sync();
         }
-        _thd_ctx.fwd_on = 0u;
-        uint64_t held = hz::wave::ballot(_thd_ctx.fwd_op != hz::LINK_NONE);
-        while (held != 0ull) {
-            const uint32_t D = hz::wave::read_lane(_thd_ctx.fwd_op, (uint32_t)__builtin_ctzll(held));
-            const bool mine = _thd_ctx.fwd_op == D;
-            held &= ~hz::wave::ballot(mine);
-            if (mine) {
+        return held_lanes();
+    }
+
+    // A stash link to fill lanes from: a ready one, else the fullest open
+    // one, LINK_NONE if there is none. Unless lanes of different operations
+    // run together, only links of the held operation qualify.
+    __device__ HZ_INLINE uint32_t fill_source(uint64_t held) {
+        GroupContext& g = _grp_ctx;
+        uint32_t rm = hz::wave::first(g.ready_mask);
+        if constexpr (CHAIN_MIXED) {
+            if (rm != 0u) return pick_ready(rm);
+            uint32_t c = 0;
+            return fullest_open(c);
+        } else {
+            if (held == 0ull) {
+                if (rm != 0u) return pick_ready(rm);
+                uint32_t c = 0;
+                return fullest_open(c);
+            }
+            const uint32_t D = hz::wave::read_lane(_thd_ctx.chain_op, (uint32_t)__builtin_ctzll(held));
+            for (; rm != 0u; rm &= rm - 1u) {
+                if (hz::wave::first(g.link_op[lowest(rm)]) == D) return lowest(rm);
+            }
+            return open_link(hz::wave::first(g.open[D]));
+        }
+    }
+
+    // Fills lanes from the stash; returns the lanes that hold a promise.
+    __device__ HZ_INLINE uint64_t refill(uint64_t held) {
+        HZ_PHASE(PHASE_READ);
+        if constexpr (!CHAIN_MIXED) {
+            if (held != 0ull && hz::wave::first(_thd_ctx.feed_count) != 0u &&
+                hz::wave::read_lane(_thd_ctx.chain_op, (uint32_t)__builtin_ctzll(held)) !=
+                    hz::wave::first(_thd_ctx.feed_op)) {
+                return_feed();
+            }
+        }
+        while (~held != 0ull) {
+            if (hz::wave::first(_thd_ctx.feed_count) == 0u) {
+                const uint32_t L = fill_source(held);
+                if (L == hz::LINK_NONE) break;
+                take_feed(L);
+                _thd_ctx.chain_streak = 0u;
+            }
+            held = fill_lanes(held);
+        }
+        return held;
+    }
+
+    // Returns the promises of the `mine` lanes to the stash, by operation
+    // (every lane active). They were counted when they were queued.
+    __device__ HZ_INLINE void park(bool mine) {
+        uint64_t left = hz::wave::ballot(mine);
+        while (left != 0ull) {
+            const uint32_t D = hz::wave::read_lane(_thd_ctx.chain_op, (uint32_t)__builtin_ctzll(left));
+            const bool go = mine && _thd_ctx.chain_op == D;
+            left &= ~hz::wave::ballot(go);
+            if (go) {
                 uint32_t words[WORDS];
 #pragma unroll
-                for (uint32_t w = 0; w < WORDS; ++w) words[w] = _thd_ctx.fwd_words[w];
+                for (uint32_t w = 0; w < WORDS; ++w) words[w] = _thd_ctx.chain_words[w];
                 stash_append(D, 0u, words);
+                _thd_ctx.chain_op = hz::LINK_NONE;
             }
             hz::wave::sync();
         }
-        _thd_ctx.fwd_op = hz::LINK_NONE;
+    }
+
+    // Every lane's promise makes room for a stash link, the next one after
+    // the link the last turn ran, and is appended to the stash.
+    __device__ HZ_INLINE void take_turn() {
+        return_feed();
+        const uint32_t used = ALL_LINKS & ~hz::wave::first(_grp_ctx.free_mask);
+        if (used == 0u) return;
+        const uint32_t after = used & ~(((2u << hz::wave::first(_thd_ctx.chain_turn)) - 1u));
+        const uint32_t L = lowest(after != 0u ? after : used);
+        const uint32_t op = _thd_ctx.chain_op;
+        uint32_t words[WORDS];
+#pragma unroll
+        for (uint32_t w = 0; w < WORDS; ++w) words[w] = _thd_ctx.chain_words[w];
+        _thd_ctx.chain_op = hz::LINK_NONE;
+        take_feed(L);
+        fill_lanes(0ull);
+        const uint32_t next_op = _thd_ctx.chain_op;
+        uint32_t next[WORDS];
+#pragma unroll
+        for (uint32_t w = 0; w < WORDS; ++w) {
+            next[w] = _thd_ctx.chain_words[w];
+            _thd_ctx.chain_words[w] = words[w];
+        }
+        _thd_ctx.chain_op = op;
+        park(op != hz::LINK_NONE);
+        _thd_ctx.chain_op = next_op;
+#pragma unroll
+        for (uint32_t w = 0; w < WORDS; ++w) _thd_ctx.chain_words[w] = next[w];
+        _thd_ctx.chain_turn = L;
+    }
+
+    // Evaluates, of the lanes' promises, those of operations I and above, one
+    // operation after another: a promise queued by one operation runs in the
+    // same pass if its own comes later. `done` counts the promises this lane
+    // ran (a vector register: a count of the operation's lanes costs two
+    // instructions of the scalar unit, which bounds short operations).
+    template <unsigned I>
+    __device__ HZ_INLINE void run_pass(uint32_t& done) {
+        if constexpr (I < OPS) {
+            using Op = typename hz::OpOf<I, OpSet>::type;
+            if (_thd_ctx.chain_op == I) {
+                done += 1u;
+                PromiseUnionType pu;
+                __builtin_memcpy(&pu, _thd_ctx.chain_words, sizeof(PromiseUnionType));
+                // The lane holds nothing now, so its words need not survive
+                // where it queues nothing (no select per word).
+                uint32_t none[WORDS];
+                __builtin_memcpy(_thd_ctx.chain_words, none, sizeof(none));
+                _thd_ctx.chain_op = hz::LINK_NONE;
+                pu.template rigid_eval<ProgramType, Op>(*this);
+            }
+            hz::wave::sync();
+            run_pass<I + 1>(done);
+        }
+    }
+
+    // Without CHAIN_MIXED, the lanes of the most common operation keep their
+    // promises; the others' go back to the stash.
+    __device__ HZ_INLINE uint64_t keep_one_operation(uint64_t held) {
+        uint32_t best = 0u, keep = hz::LINK_NONE;
+        for (uint64_t left = held; left != 0ull;) {
+            const uint32_t D = hz::wave::read_lane(_thd_ctx.chain_op, (uint32_t)__builtin_ctzll(left));
+            const uint64_t same = hz::wave::ballot(_thd_ctx.chain_op == D);
+            left &= ~same;
+            if (hz::wave::popc(same) > best) {
+                best = hz::wave::popc(same);
+                keep = D;
+            }
+        }
+        if (best == hz::wave::popc(held)) return held;
+        park(_thd_ctx.chain_op != hz::LINK_NONE && _thd_ctx.chain_op != keep);
+        return held_lanes();
+    }
+
+    // Runs passes over the lanes' promises (`n` lanes hold one) while enough
+    // lanes hold one, filling lanes from the feed between passes, up to about
+    // `limit` evaluations. Called with fewer than
+    // CHAIN_MIN lanes only when the group has nothing to fill the others
+    // with; it then goes on with what there is.
+    __device__ HZ_INLINE void run_chain(uint32_t n, uint32_t limit) {
+        HZ_PHASE(PHASE_EVAL);
+        const uint32_t least = n < CHAIN_MIN ? 1u : CHAIN_MIN;
+        uint32_t done = 0, starts = 0;       // this lane's promises, and its passes begun with one
+        uint32_t runs = 0;                   // uniform
+        uint32_t gone = 0, came = n;         // uniform: parked or held at the end; held at the start or filled
+        _thd_ctx.chain_on = 1u;
+        do {
+#pragma unroll
+            for (uint32_t p = 0; p < CHAIN_PASSES; ++p) {
+                if constexpr (COUNT_FORWARDED) starts += _thd_ctx.chain_op != hz::LINK_NONE ? 1u : 0u;
+                run_pass<0>(done);
+            }
+            runs += CHAIN_PASSES * OPS;
+            uint64_t held = held_lanes();
+            n = hz::wave::popc(held);
+            if constexpr (!CHAIN_MIXED) {
+                _thd_ctx.chain_on = 0u;
+                held = keep_one_operation(held);
+                _thd_ctx.chain_on = 1u;
+                gone += n - hz::wave::popc(held);
+                n = hz::wave::popc(held);
+            }
+            if (n < CHAIN_MIN && hz::wave::first(_thd_ctx.feed_count) != 0u) {
+                bool same = true;
+                if constexpr (!CHAIN_MIXED) {
+                    same = held == 0ull || hz::wave::read_lane(_thd_ctx.chain_op, (uint32_t)__builtin_ctzll(held)) ==
+                                               hz::wave::first(_thd_ctx.feed_op);
+                }
+                if (same) {
+                    came -= n;
+                    n = hz::wave::popc(fill_lanes(held));
+                    came += n;
+                }
+            }
+        } while (n >= least && runs < limit);
+        _thd_ctx.chain_on = 0u;
+        _thd_ctx.cycle_runs = runs;
+        _thd_ctx.chained += done;
+        _thd_ctx.runs += runs;
+        // Every promise run here was held at the start, filled from the
+        // stash or queued here, and so was every promise that is still held
+        // or was parked.
+        _thd_ctx.held += n + gone;
+        _thd_ctx.held -= came;
+        // Promises run in the pass that queued them.
+        if constexpr (COUNT_FORWARDED) _thd_ctx.forwarded += done - starts;
+        _thd_ctx.chain_streak += runs;
+    }
+
+    // Whether the group should look for more work: too few lanes hold a
+    // promise, and (unless lanes of different operations run together) no
+    // full link waits in the stash.
+    __device__ HZ_INLINE bool lanes_wanting(uint64_t held) {
+        if (hz::wave::popc(held) >= CHAIN_MIN) return false;
+        return CHAIN_MIXED || hz::wave::first(_grp_ctx.ready_mask) == 0u;
+    }
+
+    // The chaining form of a scheduling cycle up to the point where the
+    // group has nothing to run: fills lanes from the stash, then from queued
+    // links, then from new work, and runs passes. Returns true if it ran any.
+    __device__ HZ_INLINE bool chain_cycle(uint32_t pause, uint32_t left) {
+        GroupContext& g = _grp_ctx;
+        uint64_t held = held_lanes();
+        if (hz::wave::popc(held) < CHAIN_MIN) {
+            held = refill(held);
+            if constexpr (!CHAIN_MIXED) {
+                // Too few lanes of one operation: the stash coalesces them.
+                if (hz::wave::popc(held) < CHAIN_MIN && !stash_empty()) {
+                    return_feed();
+                    park(_thd_ctx.chain_op != hz::LINK_NONE);
+                    held = 0ull;
+                }
+            }
+            if (lanes_wanting(held)) {
+                // Consulting the home queue is a device-scope load, so after
+                // a check that found nothing the group runs some cycles
+                // without one; a group that holds nothing asks every time
+                // (exec_cycle).
+                const uint32_t countdown = hz::wave::first(_thd_ctx.queue_check);
+                if (countdown != 0u) {
+                    _thd_ctx.queue_check = countdown - 1u;
+                } else {
+                    HZ_PHASE(PHASE_PULL);
+                    while (lanes_wanting(held) && queues_hint() && pull_links(1) != 0u) {
+                        held = refill(held);
+                        _thd_ctx.queue_pause = 0u;
+                    }
+                    if (lanes_wanting(held)) {
+                        const uint32_t p = hz::wave::first(_thd_ctx.queue_pause) * 2u + 1u;
+                        _thd_ctx.queue_pause = hz::wave::first(g.can_make_work) || p > QUEUE_CHECK_PERIOD - 1
+                                                   ? QUEUE_CHECK_PERIOD - 1 : p;
+                        _thd_ctx.queue_check = _thd_ctx.queue_pause;
+                    }
+                }
+                HZ_PHASE(PHASE_MAKE);
+                for (uint32_t tries = 0; tries < 4 && lanes_wanting(held) && pause == 0u &&
+                                         hz::wave::first(g.can_make_work) &&
+                                         hz::wave::first(_thd_ctx.make_pause) == 0u;
+                     ++tries) {
+                    uint32_t c = hz::wave::popc(held);
+                    if constexpr (!CHAIN_MIXED) fullest_open(c);
+                    if (tries > 0 && c >= _dev_ctx.coalesce) break;
+                    make_work_step();
+                    if constexpr (CHAIN_MIXED) held = refill(held_lanes());
+                }
+            }
+            if constexpr (!CHAIN_MIXED) {
+                if (held != 0ull && hz::wave::popc(held) < CHAIN_MIN && !stash_empty()) {
+                    park(_thd_ctx.chain_op != hz::LINK_NONE);
+                    held = 0ull;
+                }
+                if (held == 0ull) held = refill(0ull);
+            }
+        }
+        if (hz::wave::first(_thd_ctx.chain_streak) >= CHAIN_TURN) {
+            take_turn();
+            held = held_lanes();
+            _thd_ctx.chain_streak = 0u;
+        }
+        if (held == 0ull) return false;
+        _thd_ctx.idle_streak = 0;
+        set_hungry(false);
+        share_links(hz::LINK_NONE);
+        run_chain(hz::wave::popc(held), left < CHAIN_RUNS / RUNS_PER_CYCLE ? left * RUNS_PER_CYCLE : CHAIN_RUNS);
+        drop_holding_if_empty();
+        return true;
     }
 
     // True if the group's home queue holds links (at some depth level).
@@ -1388,7 +1714,8 @@ class AsyncProgram {
     __device__ HZ_INLINE void share_links(uint32_t keep) {
         if constexpr (!SHARE_WORK) return;
         GroupContext& g = _grp_ctx;
-        const uint32_t others = ALL_LINKS & ~hz::wave::first(g.free_mask) & ~(1u << keep);
+        const uint32_t kept = keep < 32u ? 1u << keep : 0u;
+        const uint32_t others = ALL_LINKS & ~hz::wave::first(g.free_mask) & ~kept;
         if (others == 0) return;
         uint32_t countdown = hz::wave::first(g.share_check);
         if (hz::wave::lane() == 0) g.share_check = countdown == 0 ? SHARE_CHECK_PERIOD - 1 : countdown - 1;
@@ -1399,7 +1726,7 @@ class AsyncProgram {
         hungry = hz::wave::first(hungry);
         for (int n = 0; n < hungry; ++n) {
             uint32_t L = hz::LINK_NONE;
-            uint32_t rm = hz::wave::first(g.ready_mask) & ~(1u << keep);
+            uint32_t rm = hz::wave::first(g.ready_mask) & ~kept;
             if (rm != 0) {
                 L = lowest(rm);
             } else {
@@ -1431,17 +1758,12 @@ class AsyncProgram {
     // its first such cycle of a launch and then every QUEUE_CHECK_PERIOD-th.
     static constexpr uint32_t QUEUE_CHECK_PERIOD = 16;
 
-    __device__ HZ_INLINE CycleResult exec_cycle() {
+    // The link-by-link form (depth levels, asynchronous argument loads, or
+    // chaining turned off): picks one link, and runs it and further ready
+    // ones. Returns true if it ran any.
+    __device__ HZ_INLINE bool link_cycle(uint32_t pause) {
         GroupContext& g = _grp_ctx;
-        HZ_PHASE(PHASE_CYCLE);
-        {
-            HZ_PHASE(PHASE_SPILL);
-            spill_until_free(MARGIN);
-        }
-
         uint32_t rm = hz::wave::first(g.ready_mask);
-        const uint32_t pause = hz::wave::first(_thd_ctx.make_pause);
-        if (pause != 0u) _thd_ctx.make_pause = pause - 1u;
         if (rm == 0) {
             bool check = !hz::wave::first(g.can_make_work);
             if (!check) {
@@ -1502,9 +1824,28 @@ class AsyncProgram {
             // A group whose stash emptied stops counting as holding work once
             // per cycle, not after every link (Collatz 66.8 -> 64.5 ms).
             drop_holding_if_empty();
-            return RUN;
+            return true;
+        }
+        return false;
+    }
+
+    // `left`: cycles left of the launch's budget.
+    __device__ HZ_INLINE CycleResult exec_cycle(uint32_t left) {
+        GroupContext& g = _grp_ctx;
+        HZ_PHASE(PHASE_CYCLE);
+        {
+            HZ_PHASE(PHASE_SPILL);
+            spill_until_free(MARGIN);
         }
 
+        _thd_ctx.cycle_runs = 0u;
+        const uint32_t pause = hz::wave::first(_thd_ctx.make_pause);
+        if (pause != 0u) _thd_ctx.make_pause = pause - 1u;
+        if constexpr (CHAIN) {
+            if (chain_cycle(pause, left)) return RUN;
+        } else if (link_cycle(pause)) {
+            return RUN;
+        }
         // Nothing local: look for queued links anywhere, then test for quiescence.
         HZ_PHASE(PHASE_IDLE);
         if (pull_links(1) > 0) return RUN;
@@ -1585,8 +1926,17 @@ class AsyncProgram {
         _thd_ctx.idle_streak = 0;
         _thd_ctx.queue_check = 0;
         _thd_ctx.make_pause = 0;
-        _thd_ctx.fwd_on = 0;
-        _thd_ctx.fwd_op = hz::LINK_NONE;
+        _thd_ctx.queue_pause = 0;
+        _thd_ctx.cycle_runs = 0;
+        _thd_ctx.chain_on = 0;
+        _thd_ctx.chain_op = hz::LINK_NONE;
+        _thd_ctx.feed_link = hz::LINK_NONE;
+        _thd_ctx.feed_op = 0;
+        _thd_ctx.feed_count = 0;
+        _thd_ctx.chain_streak = 0;
+        _thd_ctx.chain_turn = 0;
+        _thd_ctx.held = 0;
+        _thd_ctx.chained = 0;
         _thd_ctx.forwarded = 0;
     }
 
@@ -1598,6 +1948,10 @@ class AsyncProgram {
         // No load into the staging block may still be in flight when the
         // workgroup's LDS is released.
         if constexpr (HAS_LAZY) __builtin_amdgcn_s_waitcnt(0);
+        if constexpr (CHAIN) {
+            return_feed();
+            park(_thd_ctx.chain_op != hz::LINK_NONE);
+        }
         if (lane == 0) {
             for (uint32_t d = 0; d < OPS * LEVELS; ++d) g.open[d] = hz::LINK_NONE;
         }
@@ -1612,10 +1966,19 @@ class AsyncProgram {
                 break;
             }
         }
-        // Sum the lanes' append counts (every lane is active here).
-        unsigned long long appended = _thd_ctx.appended;
+        // Sum the lanes' counts (every lane is active here).
+        auto sum = [](unsigned long long v) {
 #pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) appended += __shfl_xor(appended, d, 64);
+            for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+            return v;
+        };
+        unsigned long long appended = sum(_thd_ctx.appended), executed = _thd_ctx.executed, forwarded = 0;
+        if constexpr (CHAIN) {
+            const unsigned long long chained = sum(_thd_ctx.chained);
+            executed += chained;
+            appended += _thd_ctx.held + chained;
+            if constexpr (COUNT_FORWARDED) forwarded = sum(_thd_ctx.forwarded);
+        }
         if (lane == 0) {
             if (g.hungry) {
                 g.hungry = 0;
@@ -1635,10 +1998,10 @@ class AsyncProgram {
                 hz::wave::atomic_add_acqrel(&_dev_ctx.status->makers, -1);
             }
             hz::AsyncStatus* st = _dev_ctx.status;
-            hz::wave::atomic_add(&st->promises, _thd_ctx.executed);
+            hz::wave::atomic_add(&st->promises, executed);
             hz::wave::atomic_add(&st->links_run, _thd_ctx.runs);
             if (appended) hz::wave::atomic_add(&st->appended, appended);
-            if (_thd_ctx.forwarded) hz::wave::atomic_add(&st->forwarded, _thd_ctx.forwarded);
+            if (forwarded) hz::wave::atomic_add(&st->forwarded, forwarded);
             if (g.spills) hz::wave::atomic_add(&st->spills, g.spills);
             if (g.fills) hz::wave::atomic_add(&st->fills, g.fills);
             if (_thd_ctx.made) hz::wave::atomic_add(&st->make_work_calls, _thd_ctx.made);
@@ -1668,14 +2031,20 @@ class AsyncProgram {
         // The spec hooks are inlined: a hook left out of line would take the
         // program object and push the state it refers to into scratch memory.
         [[clang::always_inline]] PROGRAM_SPEC::initialize(*this);
-        for (unsigned int cycle = 0; cycle < cycle_count; ++cycle) {
-            if ((cycle & 63u) == 63u) {
+        uint32_t unchecked = 0;  // cycles since the flags were read
+        for (unsigned int left = cycle_count; left != 0u;) {
+            if (unchecked >= 63u) {
                 unsigned int flags = 0;
                 if (hz::wave::lane() == 0) flags = hz::wave::atomic_load(&_dev_ctx.status->flags);
                 flags = hz::wave::first(flags);
                 if (flags & ~COMPLETION_FLAG) break;
+                unchecked = 0;
             }
-            if (exec_cycle() == DONE) break;
+            if (exec_cycle(left) == DONE) break;
+            const uint32_t runs = hz::wave::first(_thd_ctx.cycle_runs);
+            const uint32_t spent = runs <= RUNS_PER_CYCLE ? 1u : (runs + RUNS_PER_CYCLE - 1u) / RUNS_PER_CYCLE;
+            unchecked += spent;
+            left = left > spent ? left - spent : 0u;
         }
         [[clang::always_inline]] PROGRAM_SPEC::finalize(*this);
         cleanup_runtime();

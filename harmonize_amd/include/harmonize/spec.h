@@ -60,10 +60,23 @@ HZ_CONST_OR(OLDEST_FIRST)
 // Nonzero, with STACK_SIZE depth levels: run and pull the shallowest level
 // first instead of the deepest. Not a reference constant.
 HZ_CONST_OR(SHALLOW_FIRST)
-// Zero: the async program type never forwards links (runs a link's
-// successor promises straight from registers); forwarding is on by default
-// for flat programs. Not a reference constant.
+// Zero: no lane keeps its successor promise in registers (CHAIN_LANES'
+// default), and a program that chains all the same does not count the
+// promises that run in the pass that queued them. Not a reference constant.
 HZ_CONST_OR(FORWARD_LINKS)
+// Nonzero: lanes keep their first successor promise in registers and run it
+// next (lane chaining, async.h); zero: every promise passes through the
+// stash. Defaults to FORWARD_LINKS. Not a reference constant.
+HZ_CONST_OR(CHAIN_LANES)
+// Nonzero: chaining lanes may hold different operations, which then run one
+// after another in one pass. Default for up to two operations. Not a
+// reference constant.
+HZ_CONST_OR(CHAIN_MIXED)
+// Passes over the lanes' promises between two looks at how many lanes still
+// hold one (default 1): a specification whose operations are a few
+// instructions, and whose chains are long, spares most of the looks. Not a
+// reference constant.
+HZ_CONST_OR(CHAIN_PASSES)
 #undef HZ_CONST_OR
 
 // The operation set a program type executes: the specification's OpSet, plus

@@ -127,8 +127,8 @@ struct FuturesSpec {
     static const size_t STASH_SIZE = 16;
     static const size_t FRAME_SIZE = 8;
     static const size_t POOL_SIZE = 8;
-    // Link forwarding slows the tree (2^20 leaves: 4.9 -> 8.2 ms alone,
-    // 8.5 -> 11.5 ms with 2^14 readers), so it is off here.
+    // Every end of a chain resolves a future with a release fence, which the
+    // stash spreads over a link's lanes; chaining lanes end one at a time.
     static const size_t FORWARD_LINKS = 0;
 
     template <typename PROGRAM>

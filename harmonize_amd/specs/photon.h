@@ -375,9 +375,6 @@ struct PhotonSpec {
     static const size_t POOL_SIZE = 8;
     // Four groups per workgroup share one LDS tally.
     static const size_t GROUPS_PER_BLOCK = HZ_PHOTON_BLOCK;
-    // Link forwarding (one operation, so most links would forward) costs
-    // the 1e7-photon walk 5.65 -> 6.05 ms, so it is off here.
-    static const size_t FORWARD_LINKS = 0;
 
     template <typename PROGRAM>
     __device__ static void initialize(PROGRAM prog) {

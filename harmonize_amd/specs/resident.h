@@ -500,6 +500,7 @@ struct ResidentSpecT {
     typedef ResidentClaim ThreadState;
 
     static const size_t STASH_SIZE = KIND::STASH_SIZE;
+    static const size_t CHAIN_PASSES = KIND::CHAIN_PASSES;
     static const size_t FRAME_SIZE = 8;
     static const size_t POOL_SIZE = 8;
 
@@ -583,15 +584,13 @@ __device__ HZ_INLINE void rcollatz_finish(PROGRAM& prog, unsigned int tag, unsig
     hz::resident::count_end(prog.device, prog.thread, job);
 }
 
+// As CollatzEven and CollatzOdd: starts are at least 1, and only Odd ends a
+// chain.
 struct RCollatzEven {
     using Type = void (*)(unsigned long long val, unsigned int tag, unsigned int index);
 
     template <typename PROGRAM>
     __device__ static void eval(PROGRAM prog, unsigned long long val, unsigned int tag, unsigned int index) {
-        if (val <= 1) {
-            rcollatz_finish(prog, tag, index, tag & RESIDENT_STEP_MASK);
-            return;
-        }
         rcollatz_dispatch(prog, val >> 1, tag + 1u, index);
     }
 };
@@ -601,21 +600,18 @@ struct RCollatzOdd {
 
     template <typename PROGRAM>
     __device__ static void eval(PROGRAM prog, unsigned long long val, unsigned int tag, unsigned int index) {
-        if (val <= 1) {
-            rcollatz_finish(prog, tag, index, tag & RESIDENT_STEP_MASK);
-            return;
+        const bool ends = collatz_ends(val);
+        if (collatz_apart(ends)) {
+            rcollatz_finish(prog, tag, index, val <= 1 ? tag & RESIDENT_STEP_MASK : COLLATZ_OVERFLOW);
         }
-        if (val > 0x5555555555555554ull) {
-            rcollatz_finish(prog, tag, index, COLLATZ_OVERFLOW);
-            return;
-        }
-        rcollatz_dispatch(prog, val * 3ull + 1ull, tag + 1u, index);
+        if (!ends) rcollatz_dispatch(prog, collatz_odd_step(val), tag + 1u, index);
     }
 };
 
 struct ResidentCollatzKind {
     typedef OpUnion<RCollatzEven, RCollatzOdd> OpSet;
     static const size_t STASH_SIZE = 7;
+    static const size_t CHAIN_PASSES = HZ_COLLATZ_PASSES;
 
     // One share of what is left per lane of the launch, 1 to 8 starts: a
     // large job is claimed in bulk, so claims (one atomic on the job's claim
@@ -769,9 +765,9 @@ struct RPhotonStep {
 struct ResidentPhotonKind {
     typedef OpUnion<RPhotonStep> OpSet;
     static const size_t STASH_SIZE = HZ_PHOTON_STASH;
+    static const size_t CHAIN_PASSES = 1;
 
-    // Eight photons per lane while HZ_PHOTON_SPREAD_BELOW or more are
-    // left, else one. Bulk claims also take the job's tally into LDS. (One
+    // Eight photons per lane while HZ_PHOTON_SPREAD_BELOW or more are left, else one. Bulk claims also take the job's tally into LDS. (One
     // share of what is left per lane, as for Collatz, lowers the photon
     // serving peak by a quarter; four per lane, the photon program's own
     // claim, by 6%.)

@@ -342,11 +342,15 @@ typedef struct hz_run_stats {
                                  eval, idle); zero otherwise */
     uint64_t links_run;       /* async: links evaluated; promises / links_run
                                  is the mean number of busy lanes per
-                                 evaluation (64 = perfect coalescing) */
+                                 evaluation (64 = perfect coalescing). Where
+                                 lanes chain, an operation's turn in a pass
+                                 over the lanes is an evaluation */
     uint64_t arena_links;     /* async: arena links ever taken from the bump
                                  allocator (the high-water mark of the arena) */
-    uint64_t forwarded;       /* async: promises run straight from registers by
-                                 link forwarding, bypassing the LDS stash */
+    uint64_t forwarded;       /* async: promises that ran in the same pass over
+                                 the lanes as the promise that queued them, an
+                                 operation's turn later (not counted for a
+                                 specification with FORWARD_LINKS = 0) */
 } hz_run_stats;
 
 /* Runs the Collatz program over `count` starts (d_starts may be NULL: start
