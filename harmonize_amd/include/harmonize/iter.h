@@ -93,6 +93,76 @@ struct AtomicIter {
     __device__ bool sync_done() const { return done(); }
 };
 
+// A lane's share of a claimed range: next, next + stride, ... below end.
+template <typename INDEX_TYPE>
+struct Share {
+    INDEX_TYPE next;
+    INDEX_TYPE end;
+    INDEX_TYPE stride;
+
+    HZ_HD void clear() {
+        next = 0;
+        end = 0;
+        stride = 1;
+    }
+
+    HZ_HD bool step(INDEX_TYPE& index) {
+        if (next >= end) return false;
+        index = next;
+        next += stride;
+        return true;
+    }
+};
+
+// Gives lanes whose share is used up a new one from `range`.
+//
+// On the GPU one atomic claims for the whole wavefront: per lane, what is left
+// over the launch's lanes, 1 to `most` indices. The range's counter is one
+// address for the whole device, where loads and atomics take their turn (30 ns
+// each), so a large range is claimed in large parts, and its end, or a small
+// range, one index per lane. The parts follow the counter as it is: sized
+// from a wavefront's previous claim instead, they leave too much to the last
+// few wavefronts. The lanes take the claimed indices in turn, so that a step
+// of every lane reads consecutive elements.
+template <typename INDEX_TYPE>
+__device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TYPE>& range, INDEX_TYPE most) {
+    static_assert(sizeof(INDEX_TYPE) == 4, "claims broadcast 32-bit indices");
+#if defined(__HIP_DEVICE_COMPILE__)
+    const bool need = share.next >= share.end;
+    const uint64_t lanes = hz::wave::ballot(need);
+    if (lanes == 0ull) return;
+    const INDEX_TYPE limit = range.limit;
+    const INDEX_TYPE at = (INDEX_TYPE)hz::wave::first((uint32_t)hz_load(&range.value));
+    if (at >= limit) return;
+    const INDEX_TYPE n = (INDEX_TYPE)hz::wave::popc(lanes);
+    const INDEX_TYPE r = (INDEX_TYPE)hz::wave::rank(lanes);
+    const uint64_t all = (uint64_t)gridDim.x * blockDim.x;
+    uint64_t per = (uint64_t)(limit - at) / all;
+    per = per > most ? most : per;
+    // (Near the top of the type, small claims keep the counter from wrapping.)
+    if (per < 1 || limit > (INDEX_TYPE)0xF0000000u) per = 1;
+    const INDEX_TYPE total = n * (INDEX_TYPE)per;
+    INDEX_TYPE base = 0;
+    if (need && r == 0) base = hz::wave::atomic_add(&range.value, total);
+    base = (INDEX_TYPE)hz::wave::read_lane((uint32_t)base, (uint32_t)__builtin_ctzll(lanes));
+    INDEX_TYPE end = base + total;
+    if (end < base || end > limit) end = limit;
+    if (need) {
+        share.next = base < limit ? base + r : limit;
+        share.end = end;
+        share.stride = n;
+    }
+#else
+    (void)most;
+    if (share.next >= share.end) {
+        Iter<INDEX_TYPE> it = range.leap((INDEX_TYPE)1);
+        share.next = it.value;
+        share.end = it.limit;
+        share.stride = 1;
+    }
+#endif
+}
+
 template <typename T, template <typename> class ITER_TYPE = Iter, typename INDEX_TYPE = unsigned int>
 struct ArrayIter {
     typedef INDEX_TYPE IndexType;

@@ -82,8 +82,7 @@ struct CollatzOdd {
     }
 };
 
-// Stash links per group, and start indices each thread claims from the
-// shared iterator at once (see make_work). Seven links is the smallest stash
+// Stash links per group. Seven links is the smallest stash
 // that does not spill (two open links plus the three kept free before each
 // evaluation); fewer links per wavefront mean more resident wavefronts to
 // hide LDS and memory latency: 2^26 starts take 79 ms with 7 links against
@@ -91,26 +90,14 @@ struct CollatzOdd {
 #ifndef HZ_COLLATZ_STASH
 #define HZ_COLLATZ_STASH 7
 #endif
+// Most starts a lane claims at once (claim_share).
 #ifndef HZ_COLLATZ_CLAIM
-#define HZ_COLLATZ_CLAIM 8
-#endif
-// Below this many unclaimed starts a thread claims one at a time, so that a
-// small job (or the end of a large one) spreads its chains over more
-// wavefronts: a chain advances once per scheduler cycle of its wavefront, so
-// a wavefront holding fewer chains finishes them sooner.
-#ifndef HZ_COLLATZ_SPREAD_BELOW
-#define HZ_COLLATZ_SPREAD_BELOW (1u << 22)
+#define HZ_COLLATZ_CLAIM 32
 #endif
 // Wavefront groups per workgroup.
 #ifndef HZ_COLLATZ_BLOCK
 #define HZ_COLLATZ_BLOCK 1
 #endif
-
-// Start indices a thread has claimed and not yet launched.
-struct CollatzClaim {
-    unsigned int next;
-    unsigned int end;
-};
 
 template <typename PROGRAM>
 __device__ inline void collatz_launch(PROGRAM& prog, unsigned int index) {
@@ -125,7 +112,7 @@ __device__ inline void collatz_launch(PROGRAM& prog, unsigned int index) {
 struct CollatzSpec {
     typedef OpUnion<CollatzEven, CollatzOdd> OpSet;
     typedef CollatzState DeviceState;
-    typedef CollatzClaim ThreadState;
+    typedef util::iter::Share<unsigned int> ThreadState;  // starts claimed and not yet launched
 
     static const size_t STASH_SIZE = HZ_COLLATZ_STASH;
     static const size_t GROUPS_PER_BLOCK = HZ_COLLATZ_BLOCK;
@@ -138,39 +125,25 @@ struct CollatzSpec {
 
     template <typename PROGRAM>
     __device__ static void initialize(PROGRAM prog) {
-        prog.thread.next = 0u;
-        prog.thread.end = 0u;
+        prog.thread.clear();
     }
 
     // Claimed starts not launched yet are queued now, so a pass that ends
     // early loses none of them.
     template <typename PROGRAM>
     __device__ static void finalize(PROGRAM prog) {
-        while (prog.thread.next < prog.thread.end) {
-            collatz_launch(prog, prog.thread.next);
-            prog.thread.next += 1u;
-        }
+        unsigned int index;
+        while (prog.thread.step(index)) collatz_launch(prog, index);
     }
 
     // Launches one start per thread per call, as the reference's make_work
-    // does (collaz_hrm.cpp:127-144), but claims HZ_COLLATZ_CLAIM starts from
-    // the shared iterator at a time: that iterator is one atomic counter for
-    // the whole device, and same-address atomics serialise across the XCDs.
+    // does (collaz_hrm.cpp:127-144), from the thread's share of the starts.
     template <typename PROGRAM>
     __device__ static bool make_work(PROGRAM prog) {
-        if (prog.thread.next >= prog.thread.end) {
-            util::iter::AtomicIter<unsigned int>& starts = *prog.device.iterator;
-            unsigned int at = hz_load(&starts.value);
-            unsigned int left = at < starts.limit ? starts.limit - at : 0u;
-            util::iter::Iter<unsigned int> it = starts.leap(left < HZ_COLLATZ_SPREAD_BELOW ? 1u : HZ_COLLATZ_CLAIM);
-            prog.thread.next = it.value;
-            prog.thread.end = it.limit;
-        }
-        if (prog.thread.next < prog.thread.end) {
-            collatz_launch(prog, prog.thread.next);
-            prog.thread.next += 1u;
-            return true;
-        }
-        return !prog.device.iterator->done();
+        util::iter::claim_share(prog.thread, *prog.device.iterator, (unsigned int)HZ_COLLATZ_CLAIM);
+        unsigned int index;
+        if (!prog.thread.step(index)) return false;
+        collatz_launch(prog, index);
+        return true;
     }
 };

@@ -316,33 +316,17 @@ struct PhotonStep {
     }
 };
 
-// Stash links per group, and photon ids each thread claims from the shared
-// iterator at once. make_work launches one photon per thread per call from
-// the thread's claimed block, so the shared counter (an atomic that every
-// group hits) is touched once per HZ_PHOTON_CLAIM calls. Claims of 4 took
-// the 1e7-photon walk from 5.62-5.77 ms (8) to 5.54-5.63 ms; claims of 2,
-// to 7.0 ms.
+// Stash links per group.
 #ifndef HZ_PHOTON_STASH
 #define HZ_PHOTON_STASH 4
 #endif
+// Most photons a lane claims at once (claim_share).
 #ifndef HZ_PHOTON_CLAIM
 #define HZ_PHOTON_CLAIM 4
-#endif
-// Below this many unclaimed photons a thread claims one at a time, so a
-// small job (or the end of a large one) spreads its lineages over more
-// wavefronts.
-#ifndef HZ_PHOTON_SPREAD_BELOW
-#define HZ_PHOTON_SPREAD_BELOW (1u << 17)
 #endif
 #ifndef HZ_PHOTON_BLOCK
 #define HZ_PHOTON_BLOCK 4
 #endif
-
-// Photon ids a thread has claimed and not yet launched.
-struct PhotonClaim {
-    unsigned int next;
-    unsigned int end;
-};
 
 namespace photon_detail {
 
@@ -368,7 +352,7 @@ __device__ inline void launch(PROGRAM& prog, unsigned int id) {
 struct PhotonSpec {
     typedef OpUnion<PhotonStep> OpSet;
     typedef PhotonState DeviceState;
-    typedef PhotonClaim ThreadState;
+    typedef util::iter::Share<unsigned int> ThreadState;  // ids claimed and not yet launched
 
     static const size_t STASH_SIZE = HZ_PHOTON_STASH;
     static const size_t FRAME_SIZE = 8;
@@ -378,8 +362,7 @@ struct PhotonSpec {
 
     template <typename PROGRAM>
     __device__ static void initialize(PROGRAM prog) {
-        prog.thread.next = 0u;
-        prog.thread.end = 0u;
+        prog.thread.clear();
         if (photon_detail::uses_group_tally<PROGRAM>(prog.device)) {
             double* t = photon_detail::group_tally<PROGRAM>();
             for (unsigned int i = hz_block_thread(); i < photon_detail::PHOTON_LDS_SLOTS; i += hz_block_threads()) {
@@ -394,10 +377,8 @@ struct PhotonSpec {
     // the group's device replica.
     template <typename PROGRAM>
     __device__ static void finalize(PROGRAM prog) {
-        while (prog.thread.next < prog.thread.end) {
-            photon_detail::launch(prog, prog.thread.next);
-            prog.thread.next += 1u;
-        }
+        unsigned int id;
+        while (prog.thread.step(id)) photon_detail::launch(prog, id);
         if (photon_detail::uses_group_tally<PROGRAM>(prog.device)) {
             __syncthreads();
             const double* t = photon_detail::group_tally<PROGRAM>();
@@ -412,19 +393,10 @@ struct PhotonSpec {
     // Launches one photon per thread from the origin along +z.
     template <typename PROGRAM>
     __device__ static bool make_work(PROGRAM prog) {
-        if (prog.thread.next >= prog.thread.end) {
-            util::iter::AtomicIter<unsigned int>& photons = *prog.device.iterator;
-            unsigned int at = hz_load(&photons.value);
-            unsigned int left = at < photons.limit ? photons.limit - at : 0u;
-            util::iter::Iter<unsigned int> it = photons.leap(left < HZ_PHOTON_SPREAD_BELOW ? 1u : HZ_PHOTON_CLAIM);
-            prog.thread.next = it.value;
-            prog.thread.end = it.limit;
-        }
-        if (prog.thread.next < prog.thread.end) {
-            photon_detail::launch(prog, prog.thread.next);
-            prog.thread.next += 1u;
-            return true;
-        }
-        return !prog.device.iterator->done();
+        util::iter::claim_share(prog.thread, *prog.device.iterator, (unsigned int)HZ_PHOTON_CLAIM);
+        unsigned int id;
+        if (!prog.thread.step(id)) return false;
+        photon_detail::launch(prog, id);
+        return true;
     }
 };

@@ -767,12 +767,13 @@ struct ResidentPhotonKind {
     static const size_t STASH_SIZE = HZ_PHOTON_STASH;
     static const size_t CHAIN_PASSES = 1;
 
-    // Eight photons per lane while HZ_PHOTON_SPREAD_BELOW or more are left, else one. Bulk claims also take the job's tally into LDS. (One
+    // Eight photons per lane while BULK_FROM or more are left, else one. Bulk claims also take the job's tally into LDS. (One
     // share of what is left per lane, as for Collatz, lowers the photon
     // serving peak by a quarter; four per lane, the photon program's own
     // claim, by 6%.)
+    static constexpr unsigned int BULK_FROM = 1u << 17;
     __device__ static HZ_INLINE unsigned int per_lane(unsigned int left, unsigned int) {
-        return left >= HZ_PHOTON_SPREAD_BELOW ? 8u : 1u;
+        return left >= BULK_FROM ? 8u : 1u;
     }
 
     template <typename PROGRAM>
