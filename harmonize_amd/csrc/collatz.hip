@@ -87,7 +87,7 @@ extern "C" int hz_collatz_run(int kind, const uint64_t* d_starts, uint32_t count
         CollatzState ds{(const unsigned long long*)d_starts, d_steps, iter.ptr};
 
         if (kind == HZ_ASYNC) {
-            uint32_t groups = cfg.groups ? cfg.groups : default_groups_async();
+            uint32_t groups = cfg.groups ? cfg.groups : hz::capi::groups_for<CollatzAsync>(count);
             uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
             uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
             CollatzAsync::Instance inst(arena, ds, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);

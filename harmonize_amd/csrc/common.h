@@ -56,6 +56,17 @@ int resident_groups_of() {
     return resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
 }
 
+// Groups for a program that starts from `items` items, `per_group` of them in
+// a group: no more than are resident, and none that would find no item. (An
+// idle group still checks in and out of counters that all groups share: 1,024
+// Collatz starts took 0.57 ms with 5,632 groups.)
+template <typename P>
+uint32_t groups_for(uint64_t items, uint64_t per_group = 64) {
+    const uint64_t want = items == 0 ? 1 : (items + per_group - 1) / per_group;
+    const uint64_t most = (uint64_t)resident_groups_of<P>();
+    return (uint32_t)(want < most ? want : most);
+}
+
 // Owns a device AtomicIter<unsigned int> set to [0, limit).
 struct DeviceIter {
     util::iter::AtomicIter<unsigned int>* ptr = nullptr;

@@ -127,7 +127,7 @@ extern "C" int hz_collatz_run_noalloc(const uint64_t* d_starts, uint32_t count, 
         ClaimIter* iter = (ClaimIter*)(base + OFF_ITER);
         CollatzState ds{(const unsigned long long*)d_starts, d_steps, iter};
 
-        const uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<CollatzAsync>();
+        const uint32_t groups = cfg.groups ? cfg.groups : hz::capi::groups_for<CollatzAsync>(count);
         const uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
         const unsigned int blocks = (unsigned int)blocks_for<CollatzAsync>(groups);
 

@@ -74,8 +74,8 @@ extern "C" int hz_photon_run(int kind, const hz_photon_params* params, double* d
         check(hipMemset(d_events, 0, (size_t)p.photons * sizeof(uint32_t)), "zero events");
 
         if (kind == HZ_ASYNC) {
-            uint32_t groups = cfg.groups ? cfg.groups
-                                         : (uint32_t)hz::capi::resident_groups_of<PhotonAsync>();
+            // Splits give the groups more to do than their own photons.
+            uint32_t groups = cfg.groups ? cfg.groups : hz::capi::groups_for<PhotonAsync>(p.photons, 16);
             uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
             uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
             PhotonAsync::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);

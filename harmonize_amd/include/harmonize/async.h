@@ -48,7 +48,9 @@ struct LinkQueue {
     unsigned int head;
     unsigned int pad1[31];
     int count;
-    unsigned int pad2[31];
+    unsigned int quiet;  // work queues: set once the launch has nothing left to run (beside the
+                         // count, so that an idle group reads both from one line)
+    unsigned int pad2[30];
 };
 
 // Run status and statistics of an AsyncProgram instance, kept in HBM.
@@ -427,13 +429,8 @@ class AsyncProgram {
     // safe; the wavefronts that still hold work finish it, and completion is
     // decided by the last one out.
     static constexpr uint32_t IDLE_EXIT_POLLS = 1u << 16;
-#ifndef HZ_IDLE_BACKOFF_MAX
-#define HZ_IDLE_BACKOFF_MAX 1
-#endif
-    // Longest idle pause, in units of 256 shader cycles. Growing pauses
-    // (e.g. 32) cut idle polling traffic but cost Collatz 3% (groups pick up
-    // freshly queued links later), so the default pause stays fixed.
-    static constexpr uint32_t IDLE_BACKOFF_MAX = HZ_IDLE_BACKOFF_MAX;
+    // Idle polls of which one looks at every queue and the status words.
+    static constexpr uint32_t IDLE_SCAN_PERIOD = 8;
 
     struct ThreadContext {
         unsigned int thread_id;
@@ -502,7 +499,6 @@ class AsyncProgram {
         unsigned long long int fills;
         uint32_t share_check;  // cycles until the hungry count is consulted again
         uint32_t hungry;       // this group is counted in status->hungry
-        uint32_t no_makers;    // this group has seen (and acquired) makers == 0
         uint32_t pf_link;      // stash link whose lazy values are being loaded (HAS_LAZY)
 #ifdef HZ_PHASE_TIMING
         unsigned long long int phase[8];
@@ -1191,11 +1187,11 @@ class AsyncProgram {
         }
     }
 
-    // The group joins `units` only if make_work left promises in its stash,
-    // so a call that made nothing (an idle resident program polling for
-    // jobs) costs no atomic. While make_work runs the group is still a maker,
-    // which blocks termination by itself; the units increment precedes the
-    // release that gives up the maker role.
+    // While the group is a maker it blocks termination by itself, so it joins
+    // `units` only when it gives that role up with promises left: a group
+    // whose promises run out between two make_work calls, every time, costs
+    // no atomic on the one counter that all groups share. The units increment
+    // has completed before the decrement that gives up the role is issued.
     __device__ HZ_INLINE void make_work_step() {
         GroupContext& g = _grp_ctx;
         const uint32_t lane = hz::wave::lane();
@@ -1212,14 +1208,15 @@ class AsyncProgram {
         _thd_ctx.held += hz::wave::popc(now & ~before);
         const bool holds = now != 0ull || !stash_empty();
         if (lane == 0) {
-            if (holds && !g.holding) {
-                g.holding = 1;
-                add_units(1);
-            }
             g.can_make_work = more ? 1u : 0u;
             if (!more && g.maker) {
+                if (holds && !g.holding) {
+                    g.holding = 1;
+                    add_units(1);
+                }
                 g.maker = 0;
-                hz::wave::atomic_add_acqrel(&_dev_ctx.status->makers, -1);
+                stores_done();
+                hz::wave::atomic_add(&_dev_ctx.status->makers, -1);
             }
         }
         hz::wave::sync();
@@ -1846,31 +1843,47 @@ class AsyncProgram {
         } else if (link_cycle(pause)) {
             return RUN;
         }
-        // Nothing local: look for queued links anywhere, then test for quiescence.
+        // Nothing local: look for queued links anywhere, then test for
+        // quiescence. Most polls of a group that stays idle read only its
+        // home queue's count and quiet word, which share a line: with
+        // thousands of idle groups, polling every queue and the status words
+        // each time kept those few addresses busy for a tenth of a
+        // millisecond per round.
         HZ_PHASE(PHASE_IDLE);
+        const bool maker = hz::wave::first(g.can_make_work) != 0u;
+        const uint32_t streak = hz::wave::first(_thd_ctx.idle_streak);
+        if (!maker && streak % IDLE_SCAN_PERIOD != 0u) {
+            hz::LinkQueue* q = work_queue(hz::wave::first(g.home));
+            int count = 0;
+            unsigned int quiet = 0;
+            if (hz::wave::lane() == 0) {
+                count = hz::wave::atomic_load(&q->count);
+                quiet = hz::wave::atomic_load(&q->quiet);
+            }
+            if (hz::wave::first(quiet) != 0u) return DONE;
+            if (hz::wave::first(count) <= 0) {
+                _thd_ctx.idle += 1u;
+                _thd_ctx.idle_streak = streak + 1u;
+                __builtin_amdgcn_s_sleep(4);
+                return RUN;
+            }
+        }
         if (pull_links(1) > 0) return RUN;
-        if (hz::wave::first(g.can_make_work)) {
+        if (maker) {
             if (pause != 0u) __builtin_amdgcn_s_sleep(8);
             return RUN;
         }
         set_hungry(true);
-        uint32_t streak = hz::wave::first(_thd_ctx.idle_streak);
         if (streak >= IDLE_EXIT_POLLS) return DONE;
-        // makers only falls to zero after every maker's last units increment
-        // (its decrement is a release), so once a relaxed read of makers sees
-        // zero, one acquire makes those increments visible; from then on
-        // units is read relaxed: with no makers it can only fall, and it
-        // stays at zero once there.
+        // A maker's last units increment has completed before its decrement
+        // of makers is issued, so once makers reads zero every increment is
+        // visible: units can then only fall, and stays at zero once there.
+        // Both are read at the device's coherence point, makers first.
         int makers = 0, units = 0;
         unsigned int flags = 0;
         if (hz::wave::lane() == 0) {
-            if (!g.no_makers) {
-                makers = hz::wave::atomic_load(&_dev_ctx.status->makers);
-                if (makers == 0) {
-                    hz::wave::fence_acquire();
-                    g.no_makers = 1;
-                }
-            }
+            makers = hz::wave::atomic_load(&_dev_ctx.status->makers);
+            stores_done();
             units = hz::wave::atomic_load(&_dev_ctx.status->units);
             flags = hz::wave::atomic_load(&_dev_ctx.status->flags);
         }
@@ -1879,13 +1892,13 @@ class AsyncProgram {
         makers = hz::wave::first(makers);
         units = hz::wave::first(units);
         flags = hz::wave::first(flags);
-        if ((makers == 0 && units == 0) || (flags & ~COMPLETION_FLAG) != 0) return DONE;
-        // Pause between idle polls; each poll reads queue and status lines
-        // that busy groups update. The pause may grow with the idle streak
-        // (IDLE_BACKOFF_MAX).
-        uint32_t pauses = streak / 16u + 1u;
-        if (pauses > IDLE_BACKOFF_MAX) pauses = IDLE_BACKOFF_MAX;
-        for (uint32_t i = 0; i < pauses; ++i) __builtin_amdgcn_s_sleep(4);
+        if (makers == 0 && units == 0) {
+            const uint32_t lane = hz::wave::lane();
+            for (uint32_t q = lane; q < _dev_ctx.queue_count; q += 64u) hz::wave::atomic_store(&work_queue(q)->quiet, 1u);
+            return DONE;
+        }
+        if ((flags & ~COMPLETION_FLAG) != 0) return DONE;
+        __builtin_amdgcn_s_sleep(4);
         return RUN;
     }
 
@@ -1906,11 +1919,10 @@ class AsyncProgram {
             g.spills = g.fills = 0;
             g.share_check = 0;
             g.hungry = 0;
-            g.no_makers = 0;
 #ifdef HZ_PHASE_TIMING
             for (int i = 0; i < 8; ++i) g.phase[i] = 0;
 #endif
-            hz::wave::atomic_add_acqrel(&_dev_ctx.status->makers, 1);
+            hz::wave::atomic_add(&_dev_ctx.status->makers, 1);
         }
         hz::wave::sync();
     }
@@ -1995,11 +2007,12 @@ class AsyncProgram {
             if (g.maker) {
                 if (g.can_make_work) set_flags(EARLY_HALT_FLAG);
                 g.maker = 0;
-                hz::wave::atomic_add_acqrel(&_dev_ctx.status->makers, -1);
+                stores_done();
+                hz::wave::atomic_add(&_dev_ctx.status->makers, -1);
             }
             hz::AsyncStatus* st = _dev_ctx.status;
-            hz::wave::atomic_add(&st->promises, executed);
-            hz::wave::atomic_add(&st->links_run, _thd_ctx.runs);
+            if (executed) hz::wave::atomic_add(&st->promises, executed);
+            if (_thd_ctx.runs) hz::wave::atomic_add(&st->links_run, _thd_ctx.runs);
             if (appended) hz::wave::atomic_add(&st->appended, appended);
             if (forwarded) hz::wave::atomic_add(&st->forwarded, forwarded);
             if (g.spills) hz::wave::atomic_add(&st->spills, g.spills);
@@ -2009,10 +2022,14 @@ class AsyncProgram {
 #ifdef HZ_PHASE_TIMING
             for (int i = 0; i < 8; ++i) hz::wave::atomic_add(&st->phase_cycles[i], g.phase[i]);
 #endif
-            unsigned int order = hz::wave::atomic_add_acqrel(&st->checkout, 1u);
+            // What the last group out reads is all atomics, complete before
+            // their group's checkout is issued: no fence is needed.
+            stores_done();
+            unsigned int order = hz::wave::atomic_add(&st->checkout, 1u);
             if (order == gridDim.x * GROUPS_PER_BLOCK - 1) {
                 unsigned int old = hz::wave::atomic_and(&st->flags, ~EARLY_HALT_FLAG);
-                int units = hz::wave::atomic_load_acquire(&st->units);
+                int units = hz::wave::atomic_load(&st->units);
+                for (unsigned int q = 0; q < _dev_ctx.queue_count; ++q) hz::wave::atomic_store(&work_queue(q)->quiet, 0u);
                 if ((old & EARLY_HALT_FLAG) == 0 && units == 0) set_flags(COMPLETION_FLAG);
                 hz::wave::atomic_add(&st->launches, 1ull);
                 hz::wave::atomic_store(&st->checkout, 0u);
@@ -2390,6 +2407,7 @@ class AsyncProgram {
             ctx.queues[i].tail = 0;
             ctx.queues[i].head = 0;
             ctx.queues[i].count = 0;
+            ctx.queues[i].quiet = 0;
         }
         if (tid == 0) {
             ctx.free_queue->tail = 0;
