@@ -97,6 +97,7 @@ _SIGNATURES = {
     "harmonize_memcpy_host_to_device": (None, [_VP, _VP, ctypes.c_size_t]),
     "harmonize_memcpy_device_to_host": (None, [_VP, _VP, ctypes.c_size_t]),
     "hz_device_synchronize": (ctypes.c_int, []),
+    "hz_workspace_release": (ctypes.c_int, []),
     "hz_device_copy": (ctypes.c_int, [_VP, _VP, ctypes.c_size_t]),
     "hz_device_query": (ctypes.c_int, [ctypes.POINTER(DeviceFacts)]),
     "hz_collatz_run": (
@@ -229,6 +230,11 @@ def device_copy(dst: "DeviceArray", src: "DeviceArray", nbytes: int) -> None:
     if nbytes > min(dst.nbytes, src.nbytes):
         raise ValueError("device_copy: nbytes exceeds an array")
     check(lib().hz_device_copy(dst.ptr, src.ptr, nbytes), "hz_device_copy")
+
+
+def workspace_release() -> None:
+    """Frees the device workspaces that finished runs left for later ones."""
+    check(lib().hz_workspace_release(), "hz_workspace_release")
 
 
 def device_facts() -> dict:

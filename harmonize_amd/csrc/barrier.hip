@@ -1,5 +1,5 @@
 // Remapping-barrier program of the C ABI: AsyncProgram over BarrierDemoSpec.
-#include "common.h"
+#include "workspace.h"
 #include "barrier_demo.h"
 
 using BarrierAsync = AsyncProgram<BarrierDemoSpec>;
@@ -37,13 +37,10 @@ extern "C" int hz_barrier_run(uint32_t dep_count, uint32_t non_dep_count, uint32
         check(hipMemset(d_counter, 0, sizeof(uint32_t)), "zero counter");
         check(hipMemset(d_violations, 0, sizeof(uint32_t)), "zero violations");
         if (dep_count) check(hipMemset(d_hits, 0, (size_t)dep_count * sizeof(uint32_t)), "zero hits");
-        hz::capi::DeviceIter iter(dep_count + non_dep_count);
-
         BarrierDemoState st{};
         st.dep_count = dep_count;
         st.non_dep_count = non_dep_count;
         st.barrier_count = barrier_count;
-        st.source_id_iter = iter.ptr;
         st.counter = d_counter;
         st.hits = d_hits;
         st.violations = d_violations;
@@ -51,11 +48,9 @@ extern "C" int hz_barrier_run(uint32_t dep_count, uint32_t non_dep_count, uint32
 
         uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<BarrierAsync>();
         uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
-        uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-        BarrierAsync::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-        init<BarrierAsync>(inst, groups);
-        check(hipDeviceSynchronize(), "init");
-        hz::capi::run_async<BarrierAsync>(inst, groups, cycles, cfg.max_launches, stats,
-                                          (cfg.flags & HZ_RUN_AUDIT) != 0, true);
+        hz::capi::Lease<hz::capi::AsyncSpace<BarrierAsync>> ws(arena, cfg.queues);
+        st.source_id_iter = ws->parts.set_iter(dep_count + non_dep_count);
+        ws->begin(st, cfg, groups);
+        ws->run(groups, cfg, stats, true);
     });
 }

@@ -9,7 +9,7 @@
 #include <tuple>
 #include <vector>
 
-#include "common.h"
+#include "workspace.h"
 #include "rmat.h"
 #include "bfs.h"
 
@@ -95,9 +95,15 @@ struct hz_bfs_batch {
     hipStream_t stream = nullptr;
     double build_ms = 0.0;
     std::map<std::vector<uint64_t>, std::unique_ptr<Runner>> runners;
+    // EventProgram's instance, kept like the async runners: its queues hold
+    // gigabytes for a large batch, which cost 1.5 ms or, after an idle spell,
+    // a hundred to allocate and free on every search.
+    std::unique_ptr<BfsEvent::Instance> event_instance;
+    uint64_t event_io = 0;
 
     ~hz_bfs_batch() {
         runners.clear();
+        event_instance.reset();
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -269,7 +275,14 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
         if (io < (1ull << 20)) io = 1ull << 20;
         if (io > (1ull << 30)) io = 1ull << 30;
     }
-    BfsEvent::Instance inst(io, b.state(default_split(c)));
+    if (!b.event_instance || b.event_io != io) {
+        b.event_instance.reset();
+        b.event_instance = std::make_unique<BfsEvent::Instance>(io, b.state(default_split(c)));
+        b.event_io = io;
+    }
+    BfsEvent::Instance& inst = *b.event_instance;
+    inst.device_state = b.state(default_split(c));
+    inst.reset(b.stream);
     // 16 groups per CU: measured 22.2 ms on the 64-graph batch against 23.7
     // with 32 per CU and 23.9 with 8 per CU.
     uint32_t groups = c.groups ? c.groups : (uint32_t)(hz::capi::compute_units() * 16);
@@ -488,7 +501,21 @@ extern "C" int hz_bfs_batch_run(hz_bfs_batch* batch, int kind, const hz_run_conf
         } else if (kind == HZ_ASYNC) {
             auto key = runner_key(c);
             auto it = batch->runners.find(key);
-            if (it == batch->runners.end()) it = batch->runners.emplace(key, make_async_runner(*batch, c)).first;
+            if (it == batch->runners.end()) {
+                std::unique_ptr<Runner> made;
+                try {
+                    made = make_async_runner(*batch, c);
+                } catch (const std::invalid_argument&) {
+                    throw;
+                } catch (const std::exception&) {
+                    // Room taken by what earlier runs left behind.
+                    (void)hipGetLastError();
+                    if (hz::capi::workspace_release() == 0 && !batch->event_instance) throw;
+                    batch->event_instance.reset();
+                    made = make_async_runner(*batch, c);
+                }
+                it = batch->runners.emplace(key, std::move(made)).first;
+            }
             it->second->run(stats, (c.flags & HZ_RUN_AUDIT) != 0);
         } else {
             throw std::invalid_argument("hz_bfs_batch_run: kind must be HZ_EVENT or HZ_ASYNC");
@@ -500,5 +527,6 @@ extern "C" int hz_bfs_batch_release(hz_bfs_batch* batch) {
     return guarded([&] {
         check_batch(batch);
         batch->runners.clear();
+        batch->event_instance.reset();
     });
 }

@@ -2,7 +2,7 @@
 // pointer chasing with the node as a LazyLoad argument, loaded ahead of the
 // link that consumes it (ChaseLazySpec), or read where the promise is built
 // (ChaseEagerSpec), under AsyncProgram or EventProgram.
-#include "common.h"
+#include "workspace.h"
 #include "chase.h"
 
 using hz::capi::check;
@@ -23,11 +23,10 @@ template <typename P>
 void run_async_chase(ChaseState st, const hz_run_config& cfg, hz_run_stats* stats) {
     uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<P>();
     uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
-    uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-    typename P::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-    init<P>(inst, groups);
-    check(hipDeviceSynchronize(), "init");
-    hz::capi::run_async<P>(inst, groups, cycles, cfg.max_launches, stats, (cfg.flags & HZ_RUN_AUDIT) != 0);
+    hz::capi::Lease<hz::capi::AsyncSpace<P>> ws(arena, cfg.queues);
+    st.list_iter = ws->parts.set_iter(st.lists);
+    ws->begin(st, cfg, groups);
+    ws->run(groups, cfg, stats);
 }
 
 template <typename P>
@@ -38,8 +37,9 @@ void run_event_chase(ChaseState st, uint32_t lists, const hz_run_config& cfg, hz
         io = 1ull << 16;
         while (io < 2ull * lists && io < (1ull << 26)) io <<= 1;
     }
-    typename P::Instance inst(io, st);
-    hz::capi::run_event<P>(inst, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
+    hz::capi::Lease<hz::capi::EventSpace<P>> ws(io, 0);
+    st.list_iter = ws->parts.set_iter(lists);
+    ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
 }
 
 }  // namespace
@@ -54,8 +54,7 @@ extern "C" int hz_chase_run(int kind, int lazy, uint32_t lists, const uint32_t* 
         if (config) cfg = *config;
         if (stats) std::memset(stats, 0, sizeof(*stats));
         if (lists == 0) return;
-        hz::capi::DeviceIter iter(lists);
-        ChaseState st{lists, 0u, d_heads, (const ChaseNode*)d_nodes, (unsigned long long*)d_sums, d_lengths, iter.ptr};
+        ChaseState st{lists, 0u, d_heads, (const ChaseNode*)d_nodes, (unsigned long long*)d_sums, d_lengths, nullptr};
         if (kind == HZ_ASYNC) {
             if (lazy) {
                 run_async_chase<ChaseLazyAsync>(st, cfg, stats);

@@ -2,7 +2,7 @@
 // CollatzSpec, the one-thread-per-start comparison kernel (the analogue of
 // the reference's examples/cpp/collaz/collaz_std.cpp:5-23), and the seeded
 // start generator.
-#include "common.h"
+#include "workspace.h"
 #include "collatz.h"
 #include "philox.h"
 #include "collatz_kernels.h"
@@ -83,18 +83,15 @@ extern "C" int hz_collatz_run(int kind, const uint64_t* d_starts, uint32_t count
             return;
         }
 
-        hz::capi::DeviceIter iter(count);
-        CollatzState ds{(const unsigned long long*)d_starts, d_steps, iter.ptr};
+        CollatzState ds{(const unsigned long long*)d_starts, d_steps, nullptr};
 
         if (kind == HZ_ASYNC) {
             uint32_t groups = cfg.groups ? cfg.groups : hz::capi::groups_for<CollatzAsync>(count);
             uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
-            uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-            CollatzAsync::Instance inst(arena, ds, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-            init<CollatzAsync>(inst, groups);
-            check(hipDeviceSynchronize(), "init");
-            hz::capi::run_async<CollatzAsync>(inst, groups, cycles, cfg.max_launches, stats,
-                                              (cfg.flags & HZ_RUN_AUDIT) != 0);
+            hz::capi::Lease<hz::capi::AsyncSpace<CollatzAsync>> ws(arena, cfg.queues);
+            ds.iterator = ws->parts.set_iter(count);
+            ws->begin(ds, cfg, groups);
+            ws->run(groups, cfg, stats);
         } else if (kind == HZ_EVENT) {
             uint32_t groups = cfg.groups ? cfg.groups : default_groups_event();
             uint64_t io = cfg.arena;
@@ -103,8 +100,9 @@ extern "C" int hz_collatz_run(int kind, const uint64_t* d_starts, uint32_t count
                 while (io < count && io < (1ull << 26)) io <<= 1;
             }
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
-            CollatzEvent::Instance inst(io, ds);
-            hz::capi::run_event<CollatzEvent>(inst, groups, chunk, cfg.max_launches, stats);
+            hz::capi::Lease<hz::capi::EventSpace<CollatzEvent>> ws(io, 0);
+            ds.iterator = ws->parts.set_iter(count);
+            ws->run(ds, groups, chunk, cfg.max_launches, stats);
         } else {
             throw std::invalid_argument("hz_collatz_run: unknown program kind");
         }

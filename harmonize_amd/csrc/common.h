@@ -4,6 +4,7 @@
 
 #include <harmonize.h>
 
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <string>
@@ -50,10 +51,19 @@ int resident_groups(K kernel, int block_threads = 64) {
     return per_cu * compute_units() * (block_threads / 64);
 }
 
-// The same for a program type's exec kernel.
+// The same for a program type's exec kernel (asked once per device).
 template <typename P>
 int resident_groups_of() {
-    return resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
+    static std::atomic<int> known[64];
+    int dev = 0;
+    check(hipGetDevice(&dev), "hipGetDevice");
+    if (dev < 0 || dev >= 64) return resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
+    int n = known[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        n = resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
+        known[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 // Groups for a program that starts from `items` items, `per_group` of them in
@@ -94,75 +104,24 @@ struct EventTimer {
         (void)hipEventDestroy(b);
     }
     void start() { check(hipEventRecord(a, nullptr), "hipEventRecord"); }
-    double stop() {
-        check(hipEventRecord(b, nullptr), "hipEventRecord");
+    // The span's end, if no later mark() moves it.
+    void mark() { check(hipEventRecord(b, nullptr), "hipEventRecord"); }
+    double elapsed() {
         check(hipEventSynchronize(b), "hipEventSynchronize");
         float ms = 0;
         check(hipEventElapsedTime(&ms, a, b), "hipEventElapsedTime");
         return ms;
     }
-};
-
-// Runs an AsyncProgram instance to completion: exec launches until complete().
-// With `audit`, the instance's queues and arena are audited after every
-// launch (Instance::audit) and the number of audits is reported.
-template <typename P>
-void run_async(typename P::Instance& inst, uint32_t groups, uint32_t cycles, uint32_t max_launches,
-               hz_run_stats* stats, bool audit = false, bool barriers = false) {
-    EventTimer t;
-    t.start();
-    uint64_t launches = 0;
-    uint64_t last_progress = ~0ull;
-    uint32_t audits = 0;
-    do {
-        if (max_launches && launches >= max_launches) {
-            throw std::runtime_error("AsyncProgram: launch bound reached before completion");
-        }
-        exec<P>(inst, groups, cycles);
-        check(hipGetLastError(), "exec launch");
-        check(hipDeviceSynchronize(), "exec");
-        launches++;
-        const bool done = inst.complete();  // raises on a runtime error first
-        if (audit) {
-            hz::AsyncCensus c = inst.audit(barriers);
-            audits++;
-            if (done && (c.queued_links != 0 || c.held_links != 0)) {
-                throw std::runtime_error("AsyncProgram audit: complete with links still queued or held");
-            }
-        }
-        if (done) break;
-        // A launch that evaluated no promise signals lost accounting rather
-        // than unfinished work: report it instead of looping.
-        hz::AsyncStatus s = inst.read_status();
-        uint64_t progress = s.promises;
-        if (progress == last_progress) {
-            throw std::runtime_error("AsyncProgram: a launch made no progress before completion");
-        }
-        last_progress = progress;
-    } while (true);
-    double ms = t.stop();
-    if (stats) {
-        hz::AsyncStatus s = inst.read_status();
-        stats->promises = s.promises;
-        stats->launches = launches;
-        stats->spills = s.spills;
-        stats->fills = s.fills;
-        stats->make_work_calls = s.make_work_calls;
-        stats->groups = (uint32_t)(blocks_for<P>(groups) * (P::WORK_GROUP_SIZE / 64));
-        stats->elapsed_ms = ms;
-        for (int i = 0; i < 8; ++i) stats->phase_cycles[i] = s.phase_cycles[i];
-        stats->links_run = s.links_run;
-        stats->forwarded = s.forwarded;
-        stats->audits = audits;
-        stats->arena_links = s.claim < inst.arena_size ? s.claim : inst.arena_size;
+    double stop() {
+        mark();
+        return elapsed();
     }
-}
+};
 
 // Runs an EventProgram instance generation by generation until complete().
 template <typename P>
 void run_event(typename P::Instance& inst, uint32_t groups, uint32_t chunk, uint32_t max_launches,
-               hz_run_stats* stats) {
-    EventTimer t;
+               hz_run_stats* stats, EventTimer& t) {
     t.start();
     uint64_t launches = 0;
     if (max_launches == 0) max_launches = 1u << 24;

@@ -1,5 +1,5 @@
 // Error state, device-memory helpers and device queries of the C ABI.
-#include "common.h"
+#include "workspace.h"
 
 namespace hz {
 namespace capi {
@@ -39,7 +39,14 @@ extern "C" const char* hz_last_error(void) {
 
 extern "C" void* harmonize_alloc_device_bytes(size_t size) {
     void* p = nullptr;
-    guarded([&] { check(hipMalloc(&p, size), "hipMalloc"); });
+    guarded([&] {
+        hipError_t e = hipMalloc(&p, size);
+        if (e != hipSuccess && hz::capi::workspace_release() != 0) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, size);
+        }
+        check(e, "hipMalloc");
+    });
     return p;
 }
 

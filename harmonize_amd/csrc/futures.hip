@@ -1,7 +1,7 @@
 // Futures program of the C ABI: the value-returning reduction tree of
 // specs/futures.h, under AsyncProgram (tree and readers) or EventProgram
 // (tree only: it cannot hold promises on a barrier).
-#include "common.h"
+#include "workspace.h"
 #include "futures.h"
 
 using FuturesAsync = AsyncProgram<FuturesSpec>;
@@ -56,38 +56,41 @@ extern "C" int hz_futures_run(int kind, const uint64_t* d_starts, uint32_t leave
         if (config) cfg = *config;
         if (stats) std::memset(stats, 0, sizeof(*stats));
 
-        util::host::DevBuf<unsigned long long> slot((size_t)leaves * 2u);
-        util::host::DevBuf<UnitBarrier<FuturesOps>> join((size_t)leaves);
-        util::host::DevBuf<TotalFuture> total_future((size_t)1);
-        util::host::DevBuf<UnitFuture> forwarded((size_t)(readers ? readers : 1u));
-        hz::capi::DeviceIter iter(leaves + readers);
+        // The tree's slots, joins, total and forwarded futures, on lines of their own.
+        uint64_t bytes = 0;
+        auto place = [&](uint64_t size) {
+            const uint64_t at = bytes;
+            bytes += (size + 255u) & ~255ull;
+            return at;
+        };
+        const uint64_t slot_at = place(sizeof(unsigned long long) * 2ull * leaves);
+        const uint64_t join_at = place(sizeof(UnitBarrier<FuturesOps>) * (uint64_t)leaves);
+        const uint64_t total_at = place(sizeof(TotalFuture));
+        const uint64_t forwarded_at = place(sizeof(UnitFuture) * (uint64_t)(readers ? readers : 1u));
+        hz::capi::Lease<hz::capi::Scratch> scratch(bytes, 0);
 
         FuturesState st{};
         st.starts = (const unsigned long long*)d_starts;
-        st.slot = slot.data();
-        st.join = join.data();
-        st.total = total_future.data();
-        st.forwarded = forwarded.data();
+        st.slot = (unsigned long long*)(scratch->p + slot_at);
+        st.join = (UnitBarrier<FuturesOps>*)(scratch->p + join_at);
+        st.total = (TotalFuture*)(scratch->p + total_at);
+        st.forwarded = (UnitFuture*)(scratch->p + forwarded_at);
         st.echo = (unsigned long long*)d_echo;
-        st.iter = iter.ptr;
         st.leaves = leaves;
         st.readers = readers;
 
         unsigned int setup = leaves > readers ? leaves : readers;
         hipLaunchKernelGGL(futures_setup_kernel, dim3(grid_of(setup)), dim3(256), 0, nullptr, st, setup);
         check(hipGetLastError(), "futures_setup_kernel launch");
-        check(hipDeviceSynchronize(), "futures_setup_kernel");
 
         if (kind == HZ_ASYNC) {
             uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<FuturesAsync>();
             // Held Echo and ReturnOp promises occupy arena links until the total resolves.
             uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16) + 2ull * readers / 64u + 64u;
-            uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-            FuturesAsync::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-            init<FuturesAsync>(inst, groups);
-            check(hipDeviceSynchronize(), "init");
-            hz::capi::run_async<FuturesAsync>(inst, groups, cycles, cfg.max_launches, stats,
-                                              (cfg.flags & HZ_RUN_AUDIT) != 0, true);
+            hz::capi::Lease<hz::capi::AsyncSpace<FuturesAsync>> ws(arena, cfg.queues);
+            st.iter = ws->parts.set_iter(leaves + readers);
+            ws->begin(st, cfg, groups);
+            ws->run(groups, cfg, stats, true);
         } else {
             uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<FuturesEvent>();
             uint64_t io = cfg.arena;
@@ -96,19 +99,20 @@ extern "C" int hz_futures_run(int kind, const uint64_t* d_starts, uint32_t leave
                 while (io < leaves) io <<= 1;
             }
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
-            FuturesEvent::Instance inst(io, st);
-            hz::capi::run_event<FuturesEvent>(inst, groups, chunk, cfg.max_launches, stats);
+            hz::capi::Lease<hz::capi::EventSpace<FuturesEvent>> ws(io, 0);
+            st.iter = ws->parts.set_iter(leaves + readers);
+            ws->run(st, groups, chunk, cfg.max_launches, stats);
         }
 
         TotalFuture host_total;
-        check(hipMemcpy(&host_total, total_future.data(), sizeof(TotalFuture), hipMemcpyDeviceToHost), "total");
+        check(hipMemcpy(&host_total, st.total, sizeof(TotalFuture), hipMemcpyDeviceToHost), "total");
         if (host_total.barrier.semaphore.sem != 0u) {
             throw std::runtime_error("hz_futures_run: the program completed without resolving the total");
         }
         *total = host_total.data;
         if (readers) {
             hipLaunchKernelGGL(futures_collect_kernel, dim3(grid_of(readers)), dim3(256), 0, nullptr,
-                               (const UnitFuture*)forwarded.data(), readers, (unsigned long long*)d_forwarded);
+                               (const UnitFuture*)st.forwarded, readers, (unsigned long long*)d_forwarded);
             check(hipGetLastError(), "futures_collect_kernel launch");
             check(hipDeviceSynchronize(), "futures_collect_kernel");
         }

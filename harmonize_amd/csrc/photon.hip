@@ -1,6 +1,6 @@
 // Photon-walk programs of the C ABI: EventProgram and AsyncProgram over
 // PhotonSpec.
-#include "common.h"
+#include "workspace.h"
 #include "photon.h"
 
 using PhotonEvent = EventProgram<PhotonSpec>;
@@ -67,8 +67,7 @@ extern "C" int hz_photon_run(int kind, const hz_photon_params* params, double* d
         if (stats) std::memset(stats, 0, sizeof(*stats));
         if (p.photons == 0) return;
         if (!d_tally || !d_events) throw std::invalid_argument("hz_photon_run: null tally or events");
-        hz::capi::DeviceIter iter(p.photons);
-        PhotonState st = make_state(p, d_tally, d_events, iter.ptr);
+        PhotonState st = make_state(p, d_tally, d_events, nullptr);
         size_t tally_bytes = (size_t)p.replicas * (p.bins + HZ_PHOTON_EXTRA_SLOTS) * sizeof(double);
         check(hipMemset(d_tally, 0, tally_bytes), "zero tally");
         check(hipMemset(d_events, 0, (size_t)p.photons * sizeof(uint32_t)), "zero events");
@@ -77,12 +76,10 @@ extern "C" int hz_photon_run(int kind, const hz_photon_params* params, double* d
             // Splits give the groups more to do than their own photons.
             uint32_t groups = cfg.groups ? cfg.groups : hz::capi::groups_for<PhotonAsync>(p.photons, 16);
             uint64_t arena = cfg.arena ? cfg.arena : (1ull << 16);
-            uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-            PhotonAsync::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-            init<PhotonAsync>(inst, groups);
-            check(hipDeviceSynchronize(), "init");
-            hz::capi::run_async<PhotonAsync>(inst, groups, cycles, cfg.max_launches, stats,
-                                             (cfg.flags & HZ_RUN_AUDIT) != 0);
+            hz::capi::Lease<hz::capi::AsyncSpace<PhotonAsync>> ws(arena, cfg.queues);
+            st.iterator = ws->parts.set_iter(p.photons);
+            ws->begin(st, cfg, groups);
+            ws->run(groups, cfg, stats);
         } else if (kind == HZ_EVENT) {
             uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::compute_units() * 32u;
             uint64_t io = cfg.arena;
@@ -92,8 +89,9 @@ extern "C" int hz_photon_run(int kind, const hz_photon_params* params, double* d
                 while (io < p.photons && io < (1ull << 24)) io <<= 1;
             }
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
-            PhotonEvent::Instance inst(io, st);
-            hz::capi::run_event<PhotonEvent>(inst, groups, chunk, cfg.max_launches, stats);
+            hz::capi::Lease<hz::capi::EventSpace<PhotonEvent>> ws(io, 0);
+            st.iterator = ws->parts.set_iter(p.photons);
+            ws->run(st, groups, chunk, cfg.max_launches, stats);
         } else {
             throw std::invalid_argument("hz_photon_run: kind must be HZ_EVENT or HZ_ASYNC");
         }

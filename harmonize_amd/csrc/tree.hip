@@ -2,7 +2,7 @@
 // tree of promises run flat, deepest level first (the reference's order,
 // program/async.h:1164-1181) or shallowest level first, under AsyncProgram,
 // and flat under EventProgram.
-#include "common.h"
+#include "workspace.h"
 #include "tree.h"
 
 using hz::capi::check;
@@ -18,14 +18,13 @@ using TreeEvent = EventProgram<TreeFlatSpec>;
 static_assert(TreeDeepAsync::LEVELS == TREE_LEVELS && TreeFlatAsync::LEVELS == 1, "tree depth levels");
 
 template <typename P>
-void run_tree_async(TreeState st, const hz_run_config& cfg, hz_run_stats* stats) {
+void run_tree_async(TreeState st, uint32_t roots, const hz_run_config& cfg, hz_run_stats* stats) {
     uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::resident_groups_of<P>();
     uint64_t arena = cfg.arena ? cfg.arena : (1ull << 18);
-    uint32_t cycles = cfg.cycles ? cfg.cycles : (1u << 24);
-    typename P::Instance inst(arena, st, cfg.queues, cfg.coalesce ? cfg.coalesce : 64u);
-    init<P>(inst, groups);
-    check(hipDeviceSynchronize(), "init");
-    hz::capi::run_async<P>(inst, groups, cycles, cfg.max_launches, stats, (cfg.flags & HZ_RUN_AUDIT) != 0);
+    hz::capi::Lease<hz::capi::AsyncSpace<P>> ws(arena, cfg.queues);
+    st.root_iter = ws->parts.set_iter(roots);
+    ws->begin(st, cfg, groups);
+    ws->run(groups, cfg, stats);
 }
 
 }  // namespace
@@ -50,19 +49,19 @@ extern "C" int hz_tree_run(int kind, int order, uint32_t roots, uint32_t fanout,
         check(hipMemset(d_violations, 0, sizeof(uint32_t)), "zero violations");
         if (roots) check(hipMemset(d_leaves, 0, (size_t)roots * sizeof(uint32_t)), "zero leaves");
         if (roots == 0) return;
-        hz::capi::DeviceIter iter(roots);
-        TreeState st{roots, fanout, height, order == HZ_TREE_FLAT ? 1u : TREE_LEVELS, iter.ptr, d_leaves,
+        TreeState st{roots, fanout, height, order == HZ_TREE_FLAT ? 1u : TREE_LEVELS, nullptr, d_leaves,
                      d_violations};
         if (kind == HZ_EVENT) {
             uint32_t groups = cfg.groups ? cfg.groups : (uint32_t)hz::capi::compute_units() * 16u;
             uint64_t io = cfg.arena ? cfg.arena : (1ull << 24);
-            TreeEvent::Instance inst(io, st);
-            hz::capi::run_event<TreeEvent>(inst, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
+            hz::capi::Lease<hz::capi::EventSpace<TreeEvent>> ws(io, 0);
+            st.root_iter = ws->parts.set_iter(roots);
+            ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
         } else if (kind == HZ_ASYNC) {
             switch (order) {
-                case HZ_TREE_FLAT: run_tree_async<TreeFlatAsync>(st, cfg, stats); break;
-                case HZ_TREE_DEEPEST: run_tree_async<TreeDeepAsync>(st, cfg, stats); break;
-                default: run_tree_async<TreeShallowAsync>(st, cfg, stats); break;
+                case HZ_TREE_FLAT: run_tree_async<TreeFlatAsync>(st, roots, cfg, stats); break;
+                case HZ_TREE_DEEPEST: run_tree_async<TreeDeepAsync>(st, roots, cfg, stats); break;
+                default: run_tree_async<TreeShallowAsync>(st, roots, cfg, stats); break;
             }
         } else {
             throw std::invalid_argument("hz_tree_run: kind must be HZ_EVENT or HZ_ASYNC");

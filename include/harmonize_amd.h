@@ -745,6 +745,12 @@ int hz_device_query(hz_device_facts* facts);
 
 int hz_device_synchronize(void);
 
+/* A hz_*_run call that ends well leaves its device workspace (program
+ * instance, arena, queues) for the next call of its kind and sizes on that
+ * device; idle workspaces hold at most 1 GiB in all. This frees them now. An
+ * allocation that fails frees them by itself. */
+int hz_workspace_release(void);
+
 /* Device-to-device copy of `bytes` bytes, synchronous (used to calibrate
  * HBM byte counters against a copy of known size). */
 int hz_device_copy(void* dst, const void* src, size_t bytes);
