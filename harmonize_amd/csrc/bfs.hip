@@ -100,6 +100,7 @@ struct hz_bfs_batch {
     // a hundred to allocate and free on every search.
     std::unique_ptr<BfsEvent::Instance> event_instance;
     uint64_t event_io = 0;
+    std::unique_ptr<hz::capi::HostCell<BfsEvent::Header>> event_header;
 
     ~hz_bfs_batch() {
         runners.clear();
@@ -291,14 +292,9 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     StreamTimer t(b.stream);
     t.start();
     b.enqueue_reset();
-    uint64_t launches = 0;
-    do {
-        if (launches >= max_launches) throw std::runtime_error("EventProgram: launch bound reached before completion");
-        exec<BfsEvent>(inst, groups, chunk, b.stream);
-        check(hipGetLastError(), "bfs event launch");
-        check(hipStreamSynchronize(b.stream), "bfs event exec");
-        launches++;
-    } while (!inst.complete());
+    if (!b.event_header) b.event_header = std::make_unique<hz::capi::HostCell<BfsEvent::Header>>();
+    const uint64_t launches =
+        hz::capi::run_generations<BfsEvent>(inst, groups, chunk, max_launches, b.stream, b.event_header->p);
     double ms = t.stop();
     if (stats) {
         auto s = inst.read_status();

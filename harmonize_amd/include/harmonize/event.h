@@ -1,8 +1,8 @@
 // EventProgram<Spec>: the level-synchronous program type.
 //
 // Semantics follow the reference's program/event.h:383-518: one launch
-// evaluates one generation. Each group drains the per-operation input queues
-// in chunks; a group that finds no input calls the spec's make_work until
+// evaluates one generation. Each group evaluates its share of the
+// per-operation input queues, then calls the spec's make_work until
 // make_work returns false or an output queue is half full; then every queue
 // is flipped (outputs become the next generation's inputs). The host loops
 // `exec` until a generation produces no promises.
@@ -13,19 +13,24 @@
 //    ([op][word][capacity]), so a wavefront reads or writes 64 consecutive
 //    words per row: fully coalesced 256-byte accesses;
 //  - each operation's queue is split into SEGMENTS equal segments, each with
-//    its own counters on its own 128-byte line. A group pushes to, and first
-//    drains, its home segment (blockIdx % SEGMENTS) and moves on to other
-//    segments only when its own is full or empty. Device-scope atomics on one
-//    address serialise across the XCDs at a few tens of ns each, so a single
-//    counter per queue would cap a generation at tens of millions of pushes
-//    per second;
+//    its own counter on its own 128-byte line. A group pushes to its home
+//    segment (blockIdx % SEGMENTS) and moves on to others only when its own
+//    is full. Device-scope atomics on one address serialise across the XCDs
+//    at a few tens of ns each, so a single counter per queue would cap a
+//    generation at tens of millions of pushes per second;
 //  - an async call costs one atomic per wavefront per call site (ballot +
 //    mbcnt), not one atomic and two system fences per lane as in the
-//    reference (util/iter.h:197-214); inputs are claimed chunk*64 at a time;
+//    reference (util/iter.h:197-214);
+//  - input is not claimed at all: the flip leaves, per operation, the
+//    segments' counts and the links (64 promises) before each, and group g of
+//    G takes every G-th run of links, finding a link's segment with one
+//    ballot. Everything a group reads to find its input was written before
+//    the launch, so it comes through the XCD's L2; claim counters read and
+//    advanced at the device's coherence point took 8,192 groups 60 us to find
+//    that a generation of a thousand promises had nothing for them;
 //  - the flip runs in a one-group kernel after each generation (the
 //    reference's last group checks out through a counter that every group
-//    increments). It also publishes a bitmask of the non-empty input
-//    segments, so sparse generations do not scan every counter.
+//    increments).
 #pragma once
 
 #include "host.h"
@@ -81,27 +86,33 @@ class EventProgram {
 
     struct GroupContext {
         unsigned int toggle;
-        unsigned long long int nonempty[OPS1];
     };
 
     // Counters of one segment of one operation's queue (one 128-byte line).
     struct Segment {
-        unsigned int in_count;   // promises in this segment's input
-        unsigned int in_claim;   // input claimed so far
         unsigned int out_count;  // output slots claimed (may pass the capacity)
-        unsigned int pad[29];
+        unsigned int halt;       // operation 0's: set by halt_early for this generation
+        unsigned int pad[30];
     };
 
     // Queue counters and run status, kept in HBM.
     struct Status {
-        Segment seg[OPS1][SEGMENTS];
-        unsigned long long int nonempty[OPS1];  // bit s: input segment s is non-empty
         unsigned int toggle;
         unsigned int flags;
         unsigned int flip_count;
-        unsigned int pad;
-        unsigned long long int promises;
+        unsigned int complete_at;  // flip_count when COMPLETION was last set
+        unsigned int links[OPS1];  // input links (of 64 promises, per segment) of each operation
+        alignas(8) unsigned long long int promises;
         unsigned long long int make_work_calls;
+        alignas(128) unsigned int in_count[OPS1][SEGMENTS];  // promises in each input segment
+        unsigned int in_start[OPS1][SEGMENTS];               // input links of the operation before the segment
+        alignas(128) Segment seg[OPS1][SEGMENTS];
+    };
+
+    // The words of Status that a host loop looks at between generations.
+    struct Header {
+        unsigned int toggle, flags, flip_count, complete_at;
+        unsigned int links[OPS1];
     };
 
     struct DeviceContext {
@@ -167,19 +178,7 @@ class EventProgram {
 
         // True once a generation has produced no promises. Raises if an
         // output queue overflowed (promises would have been lost).
-        bool complete() {
-            unsigned int flags = read_flags();
-            if (flags & OVERFLOW_FLAG) {
-                throw std::runtime_error(
-                    "EventProgram: an output queue overflowed; construct the Instance with a larger io_size");
-            }
-            if (flags & USAGE_FLAG) {
-                throw std::runtime_error(
-                    "EventProgram: a Return forwarded a future that was not ready (EventProgram cannot hold "
-                    "promises on a barrier)");
-            }
-            return (flags & COMPLETION_FLAG) != 0;
-        }
+        bool complete() { return flags_complete(read_flags()); }
 
         void clear_flags() {
             unsigned int zero = 0;
@@ -194,6 +193,20 @@ class EventProgram {
 
         unsigned long long int promises() { return read_status().promises; }
     };
+
+    // What the flags of a finished generation say (Instance::complete).
+    static bool flags_complete(unsigned int flags) {
+        if (flags & OVERFLOW_FLAG) {
+            throw std::runtime_error(
+                "EventProgram: an output queue overflowed; construct the Instance with a larger io_size");
+        }
+        if (flags & USAGE_FLAG) {
+            throw std::runtime_error(
+                "EventProgram: a Return forwarded a future that was not ready (EventProgram cannot hold "
+                "promises on a barrier)");
+        }
+        return (flags & COMPLETION_FLAG) != 0;
+    }
 
     DeviceContext& _dev_ctx;
     GroupContext& _grp_ctx;
@@ -273,20 +286,6 @@ class EventProgram {
         pu.template loose_eval<ProgramType>(*this, op);
     }
 
-    // Claims up to `span` input promises of operation `op` in segment `s`.
-    __device__ bool claim(uint32_t op, uint32_t s, uint32_t span, uint32_t& base, uint32_t& end) {
-        Segment& g = segment(op, s);
-        uint32_t limit = hz::wave::first(hz::wave::atomic_load(&g.in_count));
-        if (hz::wave::first(hz::wave::atomic_load(&g.in_claim)) >= limit) return false;
-        uint32_t b = 0;
-        if (hz::wave::lane() == 0) b = hz::wave::atomic_add(&g.in_claim, span);
-        b = hz::wave::first(b);
-        if (b >= limit) return false;
-        base = s * _dev_ctx.seg_capacity + b;
-        end = s * _dev_ctx.seg_capacity + ((limit - b > span) ? b + span : limit);
-        return true;
-    }
-
    public:
     __device__ void init_program() {}
 
@@ -296,13 +295,9 @@ class EventProgram {
         _thd_ctx.thread_id = blockIdx.x * 64u + lane;
         _thd_ctx.rand_state = _thd_ctx.thread_id;
         Status* st = _dev_ctx.status;
-        if (lane == 0) {
-            _grp_ctx.toggle = hz::wave::atomic_load(&st->toggle);
-            for (uint32_t i = 0; i < OPS; ++i) _grp_ctx.nonempty[i] = hz::wave::atomic_load(&st->nonempty[i]);
-        }
+        const unsigned int in = st->toggle;
+        _grp_ctx.toggle = in;
         hz::wave::sync();
-        const unsigned int in = hz::wave::first(_grp_ctx.toggle);
-        const unsigned int span = (chunk_size == 0 ? 1u : chunk_size) * 64u;
         const uint32_t home = home_segment();
         unsigned long long made = 0;
 
@@ -310,64 +305,58 @@ class EventProgram {
         // program object and push the state it refers to into scratch memory.
         [[clang::always_inline]] PROGRAM_SPEC::initialize(*this);
 
-        while (true) {
-            // Claim a chunk: home segment first, then the other non-empty ones.
-            uint32_t op = OPS, base = 0, end = 0;
-            for (uint32_t i = 0; i < OPS && op == OPS; ++i) {
-                uint64_t live = hz::wave::first((uint64_t)_grp_ctx.nonempty[i]);
-                if (live == 0) continue;
-                if ((live >> home) & 1ull) {
-                    if (claim(i, home, span, base, end)) {
-                        op = i;
-                        break;
-                    }
-                    live &= ~(1ull << home);
-                }
-                while (live != 0) {
-                    uint32_t s = (uint32_t)__builtin_ctzll(live);
-                    if (claim(i, s, span, base, end)) {
-                        op = i;
-                        break;
-                    }
-                    live &= live - 1;
-                }
-                if (op == OPS && hz::wave::lane() == 0) _grp_ctx.nonempty[i] = 0;
-                hz::wave::sync();
-            }
-            if (op == OPS) {
-                // No input left for this group: make work until the spec says
-                // it has none or this group's output segment is half full.
-                bool more = (hz::wave::first(hz::wave::atomic_load(&st->flags)) & EARLY_HALT_FLAG) == 0;
-                while (more) {
-                    for (uint32_t i = 0; i < OPS; ++i) {
-                        uint32_t n = hz::wave::first(hz::wave::atomic_load(&segment(i, home).out_count));
-                        if (n >= _dev_ctx.seg_capacity / 2) more = false;
-                    }
-                    if (!more) break;
-                    bool mine;
-                    [[clang::always_inline]] mine = PROGRAM_SPEC::make_work(*this);
-                    more = hz::wave::ballot(mine) != 0;
-                    if (more) made++;
-                }
-                break;
-            }
-            for (uint32_t i = base + lane; i < end; i += 64u) {
-                uint32_t words[WORDS];
+        // This group's links of each operation, up to chunk_size of them in a
+        // row (fewer where the generation would leave groups without any).
+        // Operations start at different groups, so that small generations of
+        // several operations do not all fall to the same ones.
+        const uint32_t most = chunk_size == 0 ? 1u : chunk_size;
+        for (uint32_t op = 0; op < OPS; ++op) {
+            const uint32_t links = st->links[op];
+            if (links == 0u) continue;
+            const uint32_t start = st->in_start[op][lane];
+            const uint32_t count = st->in_count[op][lane];
+            uint32_t run = links / gridDim.x;
+            run = run < 1u ? 1u : (run > most ? most : run);
+            uint32_t g = blockIdx.x + op * (gridDim.x / OPS1);
+            if (g >= gridDim.x) g -= gridDim.x;
+            for (uint64_t first = (uint64_t)g * run; first < links; first += (uint64_t)gridDim.x * run) {
+                const uint32_t last = first + run < links ? (uint32_t)first + run : links;
+                for (uint32_t l = (uint32_t)first; l < last; ++l) {
+                    // The last segment that starts at or before link l holds
+                    // it: an empty segment starts where its successor does.
+                    const uint32_t s = hz::wave::popc(hz::wave::ballot(start <= l)) - 1u;
+                    const uint32_t at = (l - hz::wave::read_lane(start, s)) * 64u + lane;
+                    if (at < hz::wave::read_lane(count, s)) {
+                        const size_t i = (size_t)s * _dev_ctx.seg_capacity + at;
+                        uint32_t words[WORDS];
 #pragma unroll
-                for (uint32_t w = 0; w < WORDS; ++w) words[w] = queue_row(in, op, w)[i];
-                eval_words(op, words);
+                        for (uint32_t w = 0; w < WORDS; ++w) words[w] = queue_row(in, op, w)[i];
+                        eval_words(op, words);
+                    }
+                    hz::wave::sync();
+                }
             }
+        }
+
+        // Make work until the spec says it has none or this group's output
+        // segment is half full.
+        bool more = hz::wave::first(hz::wave::atomic_load(&segment(0, home).halt)) == 0u;
+        while (more) {
+            for (uint32_t i = 0; i < OPS; ++i) {
+                uint32_t n = hz::wave::first(hz::wave::atomic_load(&segment(i, home).out_count));
+                if (n >= _dev_ctx.seg_capacity / 2) more = false;
+            }
+            if (!more) break;
+            bool mine;
+            [[clang::always_inline]] mine = PROGRAM_SPEC::make_work(*this);
+            more = hz::wave::ballot(mine) != 0;
+            if (more) made++;
         }
 
         [[clang::always_inline]] PROGRAM_SPEC::finalize(*this);
         if (lane == 0 && made) hz::wave::atomic_add(&st->make_work_calls, made);
     }
 
-    // Flips every queue for the next generation (reference event.h:500-515,
-    // util/iter.h:437-445) and records completion when nothing was produced.
-    // Launched as one 64-lane group after each generation; lane s handles
-    // segment s of every operation.
-    static_assert(SEGMENTS == 64, "flip assigns one segment per lane");
     // Zeroes the Status struct (grid-stride over its 32-bit words).
     __device__ static void kernel_reset(DeviceContext ctx) {
         unsigned int* w = (unsigned int*)ctx.status;
@@ -377,30 +366,47 @@ class EventProgram {
         }
     }
 
+    // Flips every queue for the next generation (reference event.h:500-515,
+    // util/iter.h:437-445) and records completion when nothing was produced.
+    // Launched as one 64-lane group after each generation; lane s handles
+    // segment s of every operation.
+    static_assert(SEGMENTS == 64, "flip assigns one segment per lane");
     __device__ static void flip(DeviceContext ctx) {
         Status* st = ctx.status;
         const uint32_t lane = hz::wave::lane();
-        unsigned long long executed = 0, produced = 0;
+        unsigned long long executed = 0;
+        uint32_t produced = 0;
         for (uint32_t i = 0; i < OPS; ++i) {
             Segment& g = st->seg[i][lane];
-            uint32_t done_here = g.in_count;
-            uint32_t n = g.out_count < ctx.seg_capacity ? g.out_count : ctx.seg_capacity;
-            g.in_count = n;
-            g.in_claim = 0;
+            executed += st->in_count[i][lane];
+            const uint32_t n = g.out_count < ctx.seg_capacity ? g.out_count : ctx.seg_capacity;
             g.out_count = 0;
-            uint64_t live = hz::wave::ballot(n != 0);
-            for (uint32_t l = 0; l < 64; ++l) {
-                executed += hz::wave::read_lane(done_here, l);
-                produced += hz::wave::read_lane(n, l);
+            g.halt = 0;
+            // Links before this lane's segment: an inclusive scan, less its own.
+            const uint32_t mine = n / 64u + (n % 64u != 0u ? 1u : 0u);
+            uint32_t upto = mine;
+#pragma unroll
+            for (uint32_t d = 1; d < 64u; d <<= 1) {
+                const uint32_t below = __shfl_up(upto, d, 64);
+                if (lane >= d) upto += below;
             }
-            if (lane == 0) st->nonempty[i] = live;
+            st->in_count[i][lane] = n;
+            st->in_start[i][lane] = upto - mine;
+            const uint32_t links = hz::wave::read_lane(upto, 63u);
+            if (lane == 0) st->links[i] = links;
+            produced += links;
         }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) executed += __shfl_xor(executed, d, 64);
         if (lane == 0) {
             st->promises += executed;
             st->toggle ^= 1u;
             st->flip_count += 1;
             unsigned int flags = st->flags;
-            if (produced == 0 && (flags & EARLY_HALT_FLAG) == 0) flags |= COMPLETION_FLAG;
+            if (produced == 0 && (flags & EARLY_HALT_FLAG) == 0) {
+                if ((flags & COMPLETION_FLAG) == 0) st->complete_at = st->flip_count;
+                flags |= COMPLETION_FLAG;
+            }
             st->flags = flags & ~EARLY_HALT_FLAG;
         }
     }
@@ -434,7 +440,11 @@ class EventProgram {
         return (float)n / (float)_dev_ctx.seg_capacity;
     }
 
-    __device__ void halt_early() { set_flags(EARLY_HALT_FLAG); }
+    // Rare, so it tells every home segment: a group looks only at its own.
+    __device__ void halt_early() {
+        set_flags(EARLY_HALT_FLAG);
+        for (uint32_t s = 0; s < SEGMENTS; ++s) hz::wave::atomic_store(&segment(0, s).halt, 1u);
+    }
 
     // Promises cannot be held on a RemappingBarrier (see barrier_await).
     static constexpr bool REMAPPING_AWAIT = false;

@@ -117,7 +117,8 @@ struct Share {
 // Gives lanes whose share is used up a new one from `range`.
 //
 // On the GPU one atomic claims for the whole wavefront: per lane, what is left
-// over the launch's lanes, 1 to `most` indices. The range's counter is one
+// over the launch's lanes, 1 to `most` indices (1 once fewer than `from` are
+// left). The range's counter is one
 // address for the whole device, where loads and atomics take their turn (30 ns
 // each), so a large range is claimed in large parts, and its end, or a small
 // range, one index per lane. The parts follow the counter as it is: sized
@@ -125,13 +126,17 @@ struct Share {
 // few wavefronts. The lanes take the claimed indices in turn, so that a step
 // of every lane reads consecutive elements.
 template <typename INDEX_TYPE>
-__device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TYPE>& range, INDEX_TYPE most) {
+__device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TYPE>& range, INDEX_TYPE most,
+                                   INDEX_TYPE from = 0) {
     static_assert(sizeof(INDEX_TYPE) == 4, "claims broadcast 32-bit indices");
 #if defined(__HIP_DEVICE_COMPILE__)
     const bool need = share.next >= share.end;
     const uint64_t lanes = hz::wave::ballot(need);
     if (lanes == 0ull) return;
+    // The counter only grows, so a copy in the XCD's L2 that has passed the
+    // end settles it without a turn at the counter.
     const INDEX_TYPE limit = range.limit;
+    if (__hip_atomic_load(&range.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= limit) return;
     const INDEX_TYPE at = (INDEX_TYPE)hz::wave::first((uint32_t)hz_load(&range.value));
     if (at >= limit) return;
     const INDEX_TYPE n = (INDEX_TYPE)hz::wave::popc(lanes);
@@ -140,7 +145,7 @@ __device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TY
     uint64_t per = (uint64_t)(limit - at) / all;
     per = per > most ? most : per;
     // (Near the top of the type, small claims keep the counter from wrapping.)
-    if (per < 1 || limit > (INDEX_TYPE)0xF0000000u) per = 1;
+    if (per < 1 || limit - at < from || limit > (INDEX_TYPE)0xF0000000u) per = 1;
     const INDEX_TYPE total = n * (INDEX_TYPE)per;
     INDEX_TYPE base = 0;
     if (need && r == 0) base = hz::wave::atomic_add(&range.value, total);
@@ -154,6 +159,7 @@ __device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TY
     }
 #else
     (void)most;
+    (void)from;
     if (share.next >= share.end) {
         Iter<INDEX_TYPE> it = range.leap((INDEX_TYPE)1);
         share.next = it.value;

@@ -140,7 +140,11 @@ struct CollatzSpec {
     // does (collaz_hrm.cpp:127-144), from the thread's share of the starts.
     template <typename PROGRAM>
     __device__ static bool make_work(PROGRAM prog) {
-        util::iter::claim_share(prog.thread, *prog.device.iterator, (unsigned int)HZ_COLLATZ_CLAIM);
+        // What a group of one generation has claimed and not launched goes to
+        // its output queue when it stops, so it takes less at once.
+        constexpr bool stays = PROGRAM::PERSISTENT;
+        util::iter::claim_share(prog.thread, *prog.device.iterator, stays ? (unsigned int)HZ_COLLATZ_CLAIM : 8u,
+                                stays ? 0u : 1u << 22);
         unsigned int index;
         if (!prog.thread.step(index)) return false;
         collatz_launch(prog, index);

@@ -393,7 +393,8 @@ struct PhotonSpec {
     // Launches one photon per thread from the origin along +z.
     template <typename PROGRAM>
     __device__ static bool make_work(PROGRAM prog) {
-        util::iter::claim_share(prog.thread, *prog.device.iterator, (unsigned int)HZ_PHOTON_CLAIM);
+        util::iter::claim_share(prog.thread, *prog.device.iterator, (unsigned int)HZ_PHOTON_CLAIM,
+                                PROGRAM::PERSISTENT ? 0u : 1u << 17);
         unsigned int id;
         if (!prog.thread.step(id)) return false;
         photon_detail::launch(prog, id);
