@@ -24,9 +24,10 @@
 //    (one queue per XCD by default, selected from blockIdx % 8, since
 //    workgroups are dealt to the 8 XCDs round-robin), with
 //    stealing from other queues when a group's own queue is empty;
-//  - termination is counter-based: `units` counts groups that hold promises
-//    plus links parked in queues, `makers` counts groups whose make_work may
-//    still produce work; the run is quiescent when both are zero.
+//  - termination is counter-based: `holders` counts groups that hold
+//    promises, `makers` groups whose make_work may still produce work, and
+//    the rings' tails and heads the links parked in queues; the run is
+//    quiescent when all are zero at once.
 #pragma once
 
 #include <cstdio>
@@ -41,7 +42,8 @@
 namespace hz {
 
 // One bounded multi-producer multi-consumer ring of link ids. The three
-// counters sit on separate 128-byte lines.
+// counters sit on separate 128-byte lines. Every push draws a tail position and
+// every pop a head position, so tail - head is the number of links queued.
 struct LinkQueue {
     unsigned int tail;
     unsigned int pad0[31];
@@ -51,6 +53,8 @@ struct LinkQueue {
     unsigned int quiet;  // work queues: set once the launch has nothing left to run (beside the
                          // count, so that an idle group reads both from one line)
     unsigned int pad2[30];
+    int hungry;  // groups of this home (depth level 0) that wait for queued links (SHARE_WORK)
+    unsigned int pad3[31];
 };
 
 // Run status and statistics of an AsyncProgram instance, kept in HBM.
@@ -59,12 +63,13 @@ struct AsyncStatus {
     unsigned int stall_site;          // first bounded wait that gave up (AsyncStall)
     unsigned long long stall_detail;  // what it waited on
     unsigned int pad0[28];
-    int units;
-    unsigned int pad1[31];
+    // Groups that hold promises and are not makers (low half), and how often
+    // a group has become one (high half).
+    unsigned long long holders;
+    int units;  // queued links, written by the last group to leave a launch
+    unsigned int pad1[29];
     int makers;
     unsigned int pad2[31];
-    int hungry;  // groups with no work of their own, waiting on the queues
-    unsigned int pad4[31];
     unsigned int checkout;
     unsigned int claim;
     unsigned int pad3[30];
@@ -129,7 +134,7 @@ struct AsyncSnapshot {
     unsigned int levels = 1;
 };
 
-// Checks a snapshot: every group has left (checkout, makers and hungry are
+// Checks a snapshot: every group has left (checkout, makers, holders and hungry are
 // zero), each ring's count equals tail - head and exactly its slots in
 // [head, tail) hold link ids, no link id is queued twice or both queued and
 // free, units equals the queued links, every queued link names a valid
@@ -140,9 +145,12 @@ struct AsyncSnapshot {
 inline AsyncCensus audit_snapshot(const AsyncSnapshot& s, bool allow_held) {
     auto fail = [](const std::string& what) { throw std::runtime_error("AsyncProgram audit: " + what); };
     const AsyncStatus& st = s.status;
-    if (st.checkout != 0 || st.makers != 0 || st.hungry != 0) {
+    int hungry = 0;
+    for (const LinkQueue& q : s.queues) hungry += q.hungry != 0;
+    if (st.checkout != 0 || st.makers != 0 || (unsigned int)st.holders != 0 || hungry != 0) {
         fail("groups still checked in (checkout " + std::to_string(st.checkout) + ", makers " +
-             std::to_string(st.makers) + ", hungry " + std::to_string(st.hungry) + ")");
+             std::to_string(st.makers) + ", holders " + std::to_string((unsigned int)st.holders) + ", hungry " +
+             std::to_string(hungry) + ")");
     }
     const unsigned int cap = s.capacity;
     if (cap == 0 || (cap & (cap - 1u)) != 0 || s.slots.size() != (size_t)s.queues.size() * cap) {
@@ -270,6 +278,10 @@ class AsyncProgram {
     static_assert(GROUPS_PER_BLOCK >= 1 && GROUPS_PER_BLOCK <= 16, "GROUPS_PER_BLOCK must be in [1, 16]");
     static const size_t WORK_GROUP_SIZE = 64 * GROUPS_PER_BLOCK;
     static constexpr bool SHARE_WORK = hz::spec::SHARE_WORKOr<PROGRAM_SPEC, 0>::value != 0;
+    // Whether a group that takes a link off a queue acquires what its
+    // promises' makers have released besides the promises themselves. An
+    // acquire empties the caches that the XCD's other wavefronts read through.
+    static constexpr bool LINK_ACQUIRE = hz::spec::LINK_ACQUIREOr<PROGRAM_SPEC, 1>::value != 0;
     static constexpr bool OLDEST_FIRST = hz::spec::OLDEST_FIRSTOr<PROGRAM_SPEC, 0>::value != 0;
     // Groups live for the whole launch (specifications may keep group-level
     // partial results, e.g. LDS tallies, and flush them in finalize).
@@ -353,7 +365,10 @@ class AsyncProgram {
     static constexpr uint32_t LAZY_WORDS = lazy_words();
     static constexpr bool HAS_LAZY = LAZY_WORDS > 0;
     static_assert(LAZY_WORDS <= 16, "a LazyLoad value may span at most 16 words");
-    static constexpr uint32_t SPARES = 4;
+    // Free arena links a group keeps for its next spills. Where work grows
+    // from few seeds most links travel through the queues, and a group deals
+    // with the arena for several at once (spare_batch).
+    static constexpr uint32_t SPARES = SHARE_WORK ? 32u : 4u;
 
     // Lane chaining. While promises are evaluated, each lane's first async
     // call stays in the lane's registers and is the promise the lane runs
@@ -468,6 +483,7 @@ class AsyncProgram {
         uint32_t feed_count;
         uint32_t chain_streak;         // evaluations since a link was last taken to fill lanes (uniform)
         uint32_t chain_turn;           // stash link the last turn ran (uniform)
+        uint32_t share_next;           // queue whose hungry count is consulted next (uniform, SHARE_WORK)
         unsigned long long chained;    // promises this lane ran chaining
         // With the `chained` counts, the promises the group's lanes have held
         // (uniform; wraps below zero).
@@ -498,7 +514,7 @@ class AsyncProgram {
         unsigned long long int spills;
         unsigned long long int fills;
         uint32_t share_check;  // cycles until the hungry count is consulted again
-        uint32_t hungry;       // this group is counted in status->hungry
+        uint32_t hungry;       // this group is counted as hungry at its home queue
         uint32_t pf_link;      // stash link whose lazy values are being loaded (HAS_LAZY)
 #ifdef HZ_PHASE_TIMING
         unsigned long long int phase[8];
@@ -721,18 +737,74 @@ class AsyncProgram {
     // Memory ordering. On gfx950 an agent-scope release is an L2 write-back
     // (buffer_wbl2) and an acquire an invalidation (buffer_inv) that other
     // wavefronts on the XCD then pay for in cache misses, so the runtime
-    // orders only what carries data: a link is published by one release
-    // after its words and metadata are written, and consumed by one acquire
-    // before they are read. Counters (units, queue counts, heads, tails) are
-    // relaxed; the termination check synchronises with the makers count once
-    // it reads zero (see exec_cycle).
-    __device__ void add_units(int delta) { hz::wave::atomic_add(&_dev_ctx.status->units, delta); }
+    // orders only what carries data: a link's words and metadata are written
+    // through and waited for before its id is published, and read at the
+    // device's coherence point. Counters (holders, queue counts, heads,
+    // tails) are relaxed; the termination check orders its reads (see
+    // quiescent()).
+
+    // The group starts or stops counting as one that holds promises (one
+    // lane). Starting has completed on return; what the group queued is
+    // counted by the rings' tails before it stops.
+    __device__ HZ_INLINE void hold() {
+        _grp_ctx.holding = 1;
+        hz::wave::atomic_add(&_dev_ctx.status->holders, (1ull << 32) + 1ull);
+        stores_done();
+    }
+    __device__ HZ_INLINE void let_go() {
+        _grp_ctx.holding = 0;
+        hz::wave::atomic_add(&_dev_ctx.status->holders, ~0ull);
+    }
+
+    // Links in the work queues (every lane active).
+    __device__ HZ_INLINE unsigned long long queued_links() {
+        unsigned long long n = 0;
+        for (uint32_t r = hz::wave::lane(); r < _dev_ctx.queue_count * LEVELS; r += 64u) {
+            hz::LinkQueue* q = work_queue(r);
+            n += hz::wave::atomic_load(&q->tail) - hz::wave::atomic_load(&q->head);
+        }
+        return sum_lanes(n);
+    }
+
+    // Whether nothing is left to run: no group makes work or holds promises,
+    // and no link is queued. Only groups that make work or hold promises
+    // queue a link or take one off the head, and a group starts to hold
+    // before it does, which changes the high half of `holders` for good. So
+    // if that word reads twice the same, without holders, the queues did not
+    // change in between and what was read of them was true at once.
+    //
+    // One counter of holders and queued links together takes two atomics on
+    // one address for every link through the queues, and such atomics pass
+    // one every 30 ns (10 of the 345,000-link BFS batch's 20 ms).
+    __device__ HZ_INLINE bool quiescent() {
+        int makers = 0;
+        unsigned long long holders = 0;
+        if (hz::wave::lane() == 0) {
+            makers = hz::wave::atomic_load(&_dev_ctx.status->makers);
+            stores_done();
+            holders = hz::wave::atomic_load(&_dev_ctx.status->holders);
+        }
+        holders = hz::wave::first((uint64_t)holders);
+        if (hz::wave::first(makers) != 0 || (uint32_t)holders != 0u) return false;
+        stores_done();
+        const bool none = queued_links() == 0ull;
+        stores_done();
+        unsigned long long again = 0;
+        if (hz::wave::lane() == 0) again = hz::wave::atomic_load(&_dev_ctx.status->holders);
+        return none && hz::wave::first((uint64_t)again) == holders;
+    }
+
+    // Sum over the wavefront (every lane active).
+    __device__ static HZ_INLINE unsigned long long sum_lanes(unsigned long long v) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+        return v;
+    }
 
     // ------------------------------------------------------------ link queues
-    // Both functions are called by one lane. `publish`: store the id with
-    // release semantics (the caller has not fenced the link's data itself).
-    __device__ HZ_INLINE bool queue_push(hz::LinkQueue* q, unsigned int* slots, unsigned int id,
-                                         bool publish = true) {
+    // Both functions are called by one lane. What the link holds has been
+    // written through before it is pushed.
+    __device__ HZ_INLINE bool queue_push(hz::LinkQueue* q, unsigned int* slots, unsigned int id) {
         unsigned int t = hz::wave::atomic_add(&q->tail, 1u);
         unsigned int* slot = slots + (t & _dev_ctx.queue_mask);
         uint32_t spins = 0;
@@ -743,24 +815,21 @@ class AsyncProgram {
             }
             hz::wave::sleep_short();
         }
-        if (publish) {
-            hz::wave::atomic_store_release(slot, id);
-        } else {
-            hz::wave::atomic_store(slot, id);
-        }
+        hz::wave::atomic_store(slot, id);
         hz::wave::atomic_add(&q->count, 1);
         return true;
     }
 
-    // `consume`: acquire the link's data (the caller reads it afterwards and
-    // does not fence itself).
-    __device__ HZ_INLINE unsigned int queue_pop(hz::LinkQueue* q, unsigned int* slots, bool consume = false) {
+    // `work`: a work queue, whose links are taken by groups that count as
+    // holding promises (or as makers).
+    __device__ HZ_INLINE unsigned int queue_pop(hz::LinkQueue* q, unsigned int* slots, bool work) {
         if (hz::wave::atomic_load(&q->count) <= 0) return hz::LINK_NONE;
         int c = hz::wave::atomic_add(&q->count, -1);
         if (c <= 0) {
             hz::wave::atomic_add(&q->count, 1);
             return hz::LINK_NONE;
         }
+        if (work && !_grp_ctx.holding && !_grp_ctx.maker) hold();
         unsigned int h = hz::wave::atomic_add(&q->head, 1u);
         unsigned int* slot = slots + (h & _dev_ctx.queue_mask);
         unsigned int id;
@@ -772,7 +841,6 @@ class AsyncProgram {
             }
             hz::wave::sleep_short();
         }
-        if (consume) hz::wave::fence_acquire();
         hz::wave::atomic_store(slot, hz::LINK_NONE);
         return id;
     }
@@ -804,25 +872,71 @@ class AsyncProgram {
             g.spare_count -= 1;
             return g.spare[g.spare_count];
         }
-        unsigned int id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots);
+        const uint32_t batch = spare_batch();
+        unsigned int id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
         if (id != hz::LINK_NONE) return id;
         unsigned int claim = hz::wave::atomic_load(&_dev_ctx.status->claim);
         if (claim < _dev_ctx.links) {
-            claim = hz::wave::atomic_add(&_dev_ctx.status->claim, 1u);
-            if (claim < _dev_ctx.links) return claim;
+            claim = hz::wave::atomic_add(&_dev_ctx.status->claim, batch);
+            if (claim < _dev_ctx.links) {
+                for (uint32_t i = 1; i < batch && claim + i < _dev_ctx.links; ++i) {
+                    g.spare[g.spare_count] = claim + i;
+                    g.spare_count += 1;
+                }
+                return claim;
+            }
         }
         // Another group may have just recycled one.
-        return queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots);
+        return queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
+    }
+
+    // Links a group claims at a time and gives back at a time. With one each,
+    // the counters of the claims and of the free ring, which all groups
+    // share, bounded the 64-graph BFS batch (33.5 ms; 345,000 links through
+    // the queues, 30 ns for each atomic or load of one word): claims by four
+    // or more take 26.3 ms, and links given back by 16 as well 19.7.
+    // Groups keep at most an eighth of the arena in this way, or four links
+    // each.
+    __device__ HZ_INLINE uint32_t spare_batch() {
+        if constexpr (!SHARE_WORK) return 1u;
+        const uint32_t share = _dev_ctx.links / (16u * gridDim.x * (uint32_t)GROUPS_PER_BLOCK);
+        return share < 2u ? 1u : (share > SPARES / 2u ? SPARES / 2u : share);
     }
 
     __device__ HZ_INLINE void arena_free_lane(unsigned int id) {
         GroupContext& g = _grp_ctx;
-        if (g.spare_count < SPARES) {
+        const uint32_t batch = spare_batch();
+        const uint32_t limit = batch > 2u ? 2u * batch : 4u;
+        if (g.spare_count < limit) {
             g.spare[g.spare_count] = id;
             g.spare_count += 1;
-        } else {
-            queue_push(_dev_ctx.free_queue, _dev_ctx.free_slots, id, false);
+            return;
         }
+        give_back(batch - 1u, id);
+    }
+
+    // Queues link id and the last `more` spares as free (one lane).
+    __device__ HZ_INLINE void give_back(uint32_t more, unsigned int id) {
+        GroupContext& g = _grp_ctx;
+        hz::LinkQueue* q = _dev_ctx.free_queue;
+        const unsigned int t = hz::wave::atomic_add(&q->tail, more + 1u);
+        for (uint32_t i = 0; i <= more; ++i) {
+            unsigned int* slot = _dev_ctx.free_slots + ((t + i) & _dev_ctx.queue_mask);
+            uint32_t spins = 0;
+            while (hz::wave::atomic_load(slot) != hz::LINK_NONE) {
+                if (++spins > SLOT_SPIN_LIMIT) {
+                    stall(hz::STALL_QUEUE_PUSH, queue_detail(q, t + i));
+                    return;
+                }
+                hz::wave::sleep_short();
+            }
+            hz::wave::atomic_store(slot, id);
+            if (i < more) {
+                g.spare_count -= 1;
+                id = g.spare[g.spare_count];
+            }
+        }
+        hz::wave::atomic_add(&q->count, (int)more + 1);
     }
 
     __device__ unsigned int* arena_link(unsigned int id) { return _dev_ctx.arena + (size_t)id * (WORDS * 64u); }
@@ -874,7 +988,7 @@ class AsyncProgram {
         const uint32_t* src = &g.words[L][0];
         // The link's words and metadata go out as write-through stores
         // (agent-scope relaxed), and the wavefront waits for them before the
-        // id is published; the taker acquires before it reads them. A release
+        // id is published; the taker reads them at the coherence point. A release
         // fence here wrote back the XCD's whole L2 on every spill, which cost
         // the 64-graph BFS batch a quarter of its time (38.4-38.7 against
         // 27.9-28.9 ms).
@@ -898,9 +1012,8 @@ class AsyncProgram {
         }
         stores_done();
         if (r == 0) {
-            add_units(1);
             const uint32_t ring = ring_of(lv, g.home);
-            queue_push(work_queue(ring), work_slots(ring), id, false);
+            queue_push(work_queue(ring), work_slots(ring), id);
             g.free_mask |= (1u << L);
             g.ready_mask &= ~(1u << L);
             g.spills += 1;
@@ -947,27 +1060,42 @@ class AsyncProgram {
         for (uint32_t k = 0; k < max_links; ++k) {
             uint32_t fm = hz::wave::first(g.free_mask);
             if (fm == 0) break;
+            // Every ring's count is read at once, a ring per lane in the order
+            // of preference (level, then distance from home), and only rings
+            // that hold links are asked: one round trip, where a search with
+            // four levels of 16 rings made up to 64 in a row. (Asking the
+            // home queue or the nearest four first takes links out of level
+            // order: 78,000 more evaluations, 20.9-21.8 against 19.4 ms.)
+            const uint32_t qn = _dev_ctx.queue_count;
             unsigned int id = hz::LINK_NONE;
-            if (lane == 0) {
-                uint32_t qn = _dev_ctx.queue_count;
-                for (uint32_t li = 0; li < LEVELS && id == hz::LINK_NONE; ++li) {
-                    const uint32_t lv = level_in_order(li);
-                    for (uint32_t i = 0; i < qn && id == hz::LINK_NONE; ++i) {
-                        uint32_t q = g.home + i;
-                        if (q >= qn) q -= qn;
-                        const uint32_t ring = ring_of(lv, q);
-                        id = queue_pop(work_queue(ring), work_slots(ring));
-                    }
+            for (uint32_t from = 0; from < LEVELS * qn && id == hz::LINK_NONE; from += 64u) {
+                const uint32_t i = from + lane;
+                uint32_t ring = 0u;
+                bool some = false;
+                if (i < LEVELS * qn) {
+                    const uint32_t li = LEVELS > 1 ? i / qn : 0u;
+                    uint32_t q = hz::wave::first(g.home) + (i - li * qn);
+                    if (q >= qn) q -= qn;
+                    ring = ring_of(level_in_order(li), q);
+                    some = hz::wave::atomic_load(&work_queue(ring)->count) > 0;
+                }
+                for (uint64_t m = hz::wave::ballot(some); m != 0ull && id == hz::LINK_NONE; m &= m - 1ull) {
+                    const uint32_t pick = hz::wave::read_lane(ring, (uint32_t)__builtin_ctzll(m));
+                    if (lane == 0) id = queue_pop(work_queue(pick), work_slots(pick), true);
+                    id = hz::wave::first(id);
                 }
             }
-            id = hz::wave::first(id);
             if (id == hz::LINK_NONE) break;
-            hz::wave::fence_acquire();
+            if constexpr (LINK_ACQUIRE) {
+                hz::wave::fence_acquire();
+            } else {
+                __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            }
             uint32_t L = lowest(fm);
-            const unsigned int* src = arena_link(id);
+            unsigned int* src = arena_link(id);
 #pragma unroll
-            for (uint32_t w = 0; w < WORDS; ++w) g.words[L][w * 64u + lane] = src[w * 64u + lane];
-            uint32_t meta = hz::wave::first(_dev_ctx.link_meta[id]);
+            for (uint32_t w = 0; w < WORDS; ++w) g.words[L][w * 64u + lane] = hz::wave::atomic_load(&src[w * 64u + lane]);
+            uint32_t meta = hz::wave::first(hz::wave::atomic_load(&_dev_ctx.link_meta[id]));
             if (lane == 0) {
                 g.link_op[L] = meta & 0xFFu;
                 if constexpr (LEVELS > 1) g.link_level[L] = (meta >> 8) & 0xFFu;
@@ -977,11 +1105,6 @@ class AsyncProgram {
                 if constexpr (OLDEST_FIRST) g.link_seq[L] = g.seq++;
                 g.fills += 1;
                 arena_free_lane(id);
-                if (g.holding) {
-                    add_units(-1);
-                } else {
-                    g.holding = 1;
-                }
             }
             hz::wave::sync();
             pulled++;
@@ -1179,18 +1302,15 @@ class AsyncProgram {
     __device__ HZ_INLINE void drop_holding_if_empty() {
         GroupContext& g = _grp_ctx;
         if (stash_empty() && held_lanes() == 0ull && hz::wave::first(g.holding)) {
-            if (hz::wave::lane() == 0) {
-                g.holding = 0;
-                add_units(-1);
-            }
+            if (hz::wave::lane() == 0) let_go();
             hz::wave::sync();
         }
     }
 
     // While the group is a maker it blocks termination by itself, so it joins
-    // `units` only when it gives that role up with promises left: a group
+    // `holders` only when it gives that role up with promises left: a group
     // whose promises run out between two make_work calls, every time, costs
-    // no atomic on the one counter that all groups share. The units increment
+    // no atomic on the one counter that all groups share. The increment
     // has completed before the decrement that gives up the role is issued.
     __device__ HZ_INLINE void make_work_step() {
         GroupContext& g = _grp_ctx;
@@ -1210,10 +1330,7 @@ class AsyncProgram {
         if (lane == 0) {
             g.can_make_work = more ? 1u : 0u;
             if (!more && g.maker) {
-                if (holds && !g.holding) {
-                    g.holding = 1;
-                    add_units(1);
-                }
+                if (holds && !g.holding) hold();
                 g.maker = 0;
                 stores_done();
                 hz::wave::atomic_add(&_dev_ctx.status->makers, -1);
@@ -1691,11 +1808,12 @@ class AsyncProgram {
     // Work sharing (specifications with SHARE_WORK). A group's promises stay
     // in its LDS stash until it runs short of free links, so work that grows
     // from a few seeds (a BFS frontier) would stay with the few groups that
-    // started it. Groups without work count themselves in status->hungry; a
-    // group about to run link `keep` that holds other links consults that
-    // count every SHARE_CHECK_PERIOD cycles and spills up to that many of
-    // them (full links first, then its fullest open link) to the queues.
-    static constexpr uint32_t SHARE_CHECK_PERIOD = 4;
+    // started it. Groups without work count themselves as hungry at their
+    // home queue; a group about to run link `keep` that holds other links
+    // consults one queue's count, another each time, every SHARE_CHECK_PERIOD
+    // cycles and spills up to that many of them (full links first, then its
+    // fullest open link) to the queues.
+        static constexpr uint32_t SHARE_CHECK_PERIOD = 4;
 
     __device__ HZ_INLINE void set_hungry(bool h) {
         if constexpr (!SHARE_WORK) return;
@@ -1703,7 +1821,7 @@ class AsyncProgram {
         if ((hz::wave::first(g.hungry) != 0) == h) return;
         if (hz::wave::lane() == 0) {
             g.hungry = h ? 1u : 0u;
-            hz::wave::atomic_add(&_dev_ctx.status->hungry, h ? 1 : -1);
+            hz::wave::atomic_add(&work_queue(g.home)->hungry, h ? 1 : -1);
         }
         hz::wave::sync();
     }
@@ -1719,7 +1837,9 @@ class AsyncProgram {
         hz::wave::sync();
         if (countdown != 0) return;
         int hungry = 0;
-        if (hz::wave::lane() == 0) hungry = hz::wave::atomic_load(&_dev_ctx.status->hungry);
+        const uint32_t q = hz::wave::first(_thd_ctx.share_next);
+        _thd_ctx.share_next = q + 1u < _dev_ctx.queue_count ? q + 1u : 0u;
+        if (hz::wave::lane() == 0) hungry = hz::wave::atomic_load(&work_queue(q)->hungry);
         hungry = hz::wave::first(hungry);
         for (int n = 0; n < hungry; ++n) {
             uint32_t L = hz::LINK_NONE;
@@ -1875,24 +1995,13 @@ class AsyncProgram {
         }
         set_hungry(true);
         if (streak >= IDLE_EXIT_POLLS) return DONE;
-        // A maker's last units increment has completed before its decrement
-        // of makers is issued, so once makers reads zero every increment is
-        // visible: units can then only fall, and stays at zero once there.
-        // Both are read at the device's coherence point, makers first.
-        int makers = 0, units = 0;
         unsigned int flags = 0;
-        if (hz::wave::lane() == 0) {
-            makers = hz::wave::atomic_load(&_dev_ctx.status->makers);
-            stores_done();
-            units = hz::wave::atomic_load(&_dev_ctx.status->units);
-            flags = hz::wave::atomic_load(&_dev_ctx.status->flags);
-        }
+        if (hz::wave::lane() == 0) flags = hz::wave::atomic_load(&_dev_ctx.status->flags);
         _thd_ctx.idle += 1u;
         _thd_ctx.idle_streak = streak + 1u;
-        makers = hz::wave::first(makers);
-        units = hz::wave::first(units);
+        const bool quiet = quiescent();
         flags = hz::wave::first(flags);
-        if (makers == 0 && units == 0) {
+        if (quiet) {
             const uint32_t lane = hz::wave::lane();
             for (uint32_t q = lane; q < _dev_ctx.queue_count; q += 64u) hz::wave::atomic_store(&work_queue(q)->quiet, 1u);
             return DONE;
@@ -1945,6 +2054,7 @@ class AsyncProgram {
         _thd_ctx.feed_link = hz::LINK_NONE;
         _thd_ctx.feed_op = 0;
         _thd_ctx.feed_count = 0;
+        _thd_ctx.share_next = _grp_ctx.home;
         _thd_ctx.chain_streak = 0;
         _thd_ctx.chain_turn = 0;
         _thd_ctx.held = 0;
@@ -1978,31 +2088,25 @@ class AsyncProgram {
                 break;
             }
         }
-        // Sum the lanes' counts (every lane is active here).
-        auto sum = [](unsigned long long v) {
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-            return v;
-        };
-        unsigned long long appended = sum(_thd_ctx.appended), executed = _thd_ctx.executed, forwarded = 0;
+        // Sum the lanes' counts.
+        unsigned long long appended = sum_lanes(_thd_ctx.appended), executed = _thd_ctx.executed, forwarded = 0;
         if constexpr (CHAIN) {
-            const unsigned long long chained = sum(_thd_ctx.chained);
+            const unsigned long long chained = sum_lanes(_thd_ctx.chained);
             executed += chained;
             appended += _thd_ctx.held + chained;
-            if constexpr (COUNT_FORWARDED) forwarded = sum(_thd_ctx.forwarded);
+            if constexpr (COUNT_FORWARDED) forwarded = sum_lanes(_thd_ctx.forwarded);
         }
+        hz::AsyncStatus* st = _dev_ctx.status;
+        unsigned int order = 0;
         if (lane == 0) {
             if (g.hungry) {
                 g.hungry = 0;
-                hz::wave::atomic_add(&_dev_ctx.status->hungry, -1);
+                hz::wave::atomic_add(&work_queue(g.home)->hungry, -1);
             }
-            if (g.holding) {
-                g.holding = 0;
-                add_units(-1);
-            }
-            while (g.spare_count > 0) {
+            if (g.holding) let_go();
+            if (g.spare_count > 0) {
                 g.spare_count -= 1;
-                queue_push(_dev_ctx.free_queue, _dev_ctx.free_slots, g.spare[g.spare_count], false);
+                give_back(g.spare_count, g.spare[g.spare_count]);
             }
             if (g.maker) {
                 if (g.can_make_work) set_flags(EARLY_HALT_FLAG);
@@ -2010,7 +2114,6 @@ class AsyncProgram {
                 stores_done();
                 hz::wave::atomic_add(&_dev_ctx.status->makers, -1);
             }
-            hz::AsyncStatus* st = _dev_ctx.status;
             if (executed) hz::wave::atomic_add(&st->promises, executed);
             if (_thd_ctx.runs) hz::wave::atomic_add(&st->links_run, _thd_ctx.runs);
             if (appended) hz::wave::atomic_add(&st->appended, appended);
@@ -2025,11 +2128,14 @@ class AsyncProgram {
             // What the last group out reads is all atomics, complete before
             // their group's checkout is issued: no fence is needed.
             stores_done();
-            unsigned int order = hz::wave::atomic_add(&st->checkout, 1u);
-            if (order == gridDim.x * GROUPS_PER_BLOCK - 1) {
+            order = hz::wave::atomic_add(&st->checkout, 1u);
+        }
+        if (hz::wave::first(order) == gridDim.x * GROUPS_PER_BLOCK - 1) {
+            const int units = (int)queued_links();
+            for (uint32_t q = lane; q < _dev_ctx.queue_count; q += 64u) hz::wave::atomic_store(&work_queue(q)->quiet, 0u);
+            if (lane == 0) {
                 unsigned int old = hz::wave::atomic_and(&st->flags, ~EARLY_HALT_FLAG);
-                int units = hz::wave::atomic_load(&st->units);
-                for (unsigned int q = 0; q < _dev_ctx.queue_count; ++q) hz::wave::atomic_store(&work_queue(q)->quiet, 0u);
+                hz::wave::atomic_store(&st->units, units);
                 if ((old & EARLY_HALT_FLAG) == 0 && units == 0) set_flags(COMPLETION_FLAG);
                 hz::wave::atomic_add(&st->launches, 1ull);
                 hz::wave::atomic_store(&st->checkout, 0u);
@@ -2225,14 +2331,13 @@ class AsyncProgram {
         const unsigned int head = atomicExch(&b.full_head, hz::BARRIER_RELEASED);
         hz::wave::fence_acquire();
         // No link joins the list after the exchange, so it is counted first:
-        // one unit update covers every link before the first is queued, and
         // one tail draw places them all. The links are then placed in chunks,
         // each read off the list before any of it is queued (a queued link may
         // be reused), with the chunk's ring-slot checks issued together and
-        // one count update publishing it. (A unit update waited for, a tail
-        // draw and a slot check per link made the walk four round trips per
-        // link: 12 ms of the barrier demo at 512 links per barrier. A unit
-        // update and tail draw per chunk of four cost more than they saved.)
+        // one count update publishing it. (A tail draw and a slot check per
+        // link made the walk three round trips per link: 12 ms of the barrier
+        // demo at 512 links per barrier. A tail draw per chunk of four cost
+        // more than it saved.)
         // A chunk's ids and slot checks are held in registers: four per chunk
         // keep the barrier demo's kernel at 66 VGPRs (7 waves per SIMD), where
         // 8 and 16 take 82 and 122.
@@ -2241,9 +2346,8 @@ class AsyncProgram {
             L = hz::wave::atomic_load(&_dev_ctx.link_aux[2u * L]);
         }
         if (n == 0u) return;
-        add_units((int)n);
-        // The units, and the links' slots and metadata (written through by
-        // the lanes that filled them), are complete before any link is queued.
+        // The links' slots and metadata (written through by the lanes that
+        // filled them) are complete before any link is queued.
         stores_done();
         constexpr unsigned int CHUNK = 4;
         hz::LinkQueue* q = work_queue(_grp_ctx.home);
@@ -2302,13 +2406,13 @@ class AsyncProgram {
 
     // Any-lane arena allocation (the wave's spare cache is single-lane).
     __device__ HZ_INLINE unsigned int arena_alloc_any() {
-        unsigned int id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots);
+        unsigned int id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
         if (id != hz::LINK_NONE) return id;
         if (hz::wave::atomic_load(&_dev_ctx.status->claim) < _dev_ctx.links) {
             unsigned int claim = hz::wave::atomic_add(&_dev_ctx.status->claim, 1u);
             if (claim < _dev_ctx.links) return claim;
         }
-        return queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots);
+        return queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
     }
 
     __device__ HZ_INLINE void write_arena_slot(unsigned int L, unsigned int slot, const uint32_t* words) {
@@ -2351,9 +2455,7 @@ class AsyncProgram {
         unsigned int h = hz::wave::atomic_load(&b.full_head);
         for (uint32_t spins = 0; spins < SLOT_SPIN_LIMIT; ++spins) {
             if (h == hz::BARRIER_RELEASED) {
-                add_units(1);
-                stores_done();
-                queue_push(work_queue(_grp_ctx.home), work_slots(_grp_ctx.home), L, false);
+                queue_push(work_queue(_grp_ctx.home), work_slots(_grp_ctx.home), L);
                 return;
             }
             hz::wave::atomic_store(&_dev_ctx.link_aux[2u * L], h);
@@ -2408,18 +2510,21 @@ class AsyncProgram {
             ctx.queues[i].head = 0;
             ctx.queues[i].count = 0;
             ctx.queues[i].quiet = 0;
+            ctx.queues[i].hungry = 0;
         }
         if (tid == 0) {
             ctx.free_queue->tail = 0;
             ctx.free_queue->head = 0;
             ctx.free_queue->count = 0;
+            ctx.free_queue->quiet = 0;
+            ctx.free_queue->hungry = 0;
             hz::AsyncStatus* st = ctx.status;
             st->flags = 0;
             st->stall_site = 0;
             st->stall_detail = 0;
+            st->holders = 0;
             st->units = 0;
             st->makers = 0;
-            st->hungry = 0;
             st->checkout = 0;
             st->claim = 0;
             st->promises = st->spills = st->fills = st->make_work_calls = st->launches = st->idle_polls = 0;
