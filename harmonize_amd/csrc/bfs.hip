@@ -15,6 +15,8 @@
 
 using BfsAsync1 = AsyncProgram<BfsSpecT<1>>;
 using BfsEvent = EventProgram<BfsSpecT<1>>;
+// The batch's own programs look levels up through hints.
+using BfsEventHints = EventProgram<BfsSpecT<1, 16, true>>;
 
 static_assert(sizeof(BfsJob) == 32, "BfsJob layout");
 static_assert(sizeof(hz_bfs_state) == sizeof(BfsState), "C and C++ BFS states must match");
@@ -90,7 +92,7 @@ struct hz_bfs_batch {
     std::vector<uint32_t> vertices, sources;
     std::vector<uint64_t> edges, vertex_base, edge_base, row_base;
     uint64_t total_vertices = 0, total_edges = 0;
-    DeviceBytes row_ptr, col, level, jobs;
+    DeviceBytes row_ptr, col, level, jobs, hints;
     std::unique_ptr<hz::capi::DeviceIter> iter;
     hipStream_t stream = nullptr;
     double build_ms = 0.0;
@@ -98,9 +100,9 @@ struct hz_bfs_batch {
     // EventProgram's instance, kept like the async runners: its queues hold
     // gigabytes for a large batch, which cost 1.5 ms or, after an idle spell,
     // a hundred to allocate and free on every search.
-    std::unique_ptr<BfsEvent::Instance> event_instance;
+    std::unique_ptr<BfsEventHints::Instance> event_instance;
     uint64_t event_io = 0;
-    std::unique_ptr<hz::capi::HostCell<BfsEvent::Header>> event_header;
+    std::unique_ptr<hz::capi::HostCell<BfsEventHints::Header>> event_header;
 
     ~hz_bfs_batch() {
         runners.clear();
@@ -131,6 +133,7 @@ struct hz_bfs_batch {
         row_ptr = DeviceBytes((total_vertices + graphs) * sizeof(int32_t));
         col = DeviceBytes(total_edges * sizeof(int32_t));
         level = DeviceBytes(total_vertices * sizeof(int32_t));
+        hints = DeviceBytes((total_vertices + 7) / 8 * 4);
         jobs = DeviceBytes(graphs * sizeof(BfsJob));
         iter = std::make_unique<hz::capi::DeviceIter>(graphs);
         check(hipStreamCreate(&stream), "hipStreamCreate");
@@ -148,8 +151,10 @@ struct hz_bfs_batch {
         check(hipMemcpy(jobs.p, host.data(), graphs * sizeof(BfsJob), hipMemcpyHostToDevice), "jobs upload");
     }
 
-    BfsState state(uint32_t split) const {
-        BfsState s{};
+    BfsHintState state(uint32_t split) const {
+        BfsHintState s{};
+        s.hints = hints.as<unsigned char>();
+        s.level_base = level.as<int32_t>();
         s.jobs = jobs.as<BfsJob>();
         s.job_iter = iter->ptr;
         s.job_count = graphs;
@@ -159,7 +164,7 @@ struct hz_bfs_batch {
 
     void enqueue_reset() {
         hipLaunchKernelGGL(bfs_reset_kernel, dim3(grid_for(total_vertices)), dim3(256), 0, stream,
-                           level.as<int32_t>(), total_vertices, iter->ptr, graphs);
+                           level.as<int32_t>(), total_vertices, iter->ptr, graphs, hints.as<uint32_t>());
     }
 };
 
@@ -278,10 +283,10 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     }
     if (!b.event_instance || b.event_io != io) {
         b.event_instance.reset();
-        b.event_instance = std::make_unique<BfsEvent::Instance>(io, b.state(default_split(c)));
+        b.event_instance = std::make_unique<BfsEventHints::Instance>(io, b.state(default_split(c)));
         b.event_io = io;
     }
-    BfsEvent::Instance& inst = *b.event_instance;
+    BfsEventHints::Instance& inst = *b.event_instance;
     inst.device_state = b.state(default_split(c));
     inst.reset(b.stream);
     // 16 groups per CU: measured 22.2 ms on the 64-graph batch against 23.7
@@ -292,9 +297,9 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     StreamTimer t(b.stream);
     t.start();
     b.enqueue_reset();
-    if (!b.event_header) b.event_header = std::make_unique<hz::capi::HostCell<BfsEvent::Header>>();
+    if (!b.event_header) b.event_header = std::make_unique<hz::capi::HostCell<BfsEventHints::Header>>();
     const uint64_t launches =
-        hz::capi::run_generations<BfsEvent>(inst, groups, chunk, max_launches, b.stream, b.event_header->p);
+        hz::capi::run_generations<BfsEventHints>(inst, groups, chunk, max_launches, b.stream, b.event_header->p);
     double ms = t.stop();
     if (stats) {
         auto s = inst.read_status();
@@ -317,11 +322,11 @@ std::unique_ptr<Runner> make_async_runner_stash(hz_bfs_batch& b, const hz_run_co
     switch (c.block_groups) {
         case 0:
         case 1:
-            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<1, STASH>>>>(b, c);
+            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<1, STASH, true>>>>(b, c);
         case 2:
-            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<2, STASH>>>>(b, c);
+            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<2, STASH, true>>>>(b, c);
         case 4:
-            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<4, STASH>>>>(b, c);
+            return std::make_unique<AsyncRunner<AsyncProgram<BfsSpecT<4, STASH, true>>>>(b, c);
         default:
             throw std::invalid_argument("hz_bfs_batch_run: block_groups must be 1, 2 or 4");
     }

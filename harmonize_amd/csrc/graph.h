@@ -39,11 +39,15 @@ static __global__ void __launch_bounds__(256)
     }
 }
 
-// Levels to BFS_UNREACHED and the job iterator to [0, jobs): a kernel, so
-// that it can be captured in a graph.
+// Levels to BFS_UNREACHED, level hints (if any) to BFS_NO_HINT and the job
+// iterator to [0, jobs): a kernel, so that it can be captured in a graph.
 static __global__ void __launch_bounds__(256)
-    bfs_reset_kernel(int32_t* level, uint64_t n, util::iter::AtomicIter<unsigned int>* iter, unsigned int jobs) {
+    bfs_reset_kernel(int32_t* level, uint64_t n, util::iter::AtomicIter<unsigned int>* iter, unsigned int jobs,
+                     uint32_t* hints = nullptr) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    if (hints != nullptr) {
+        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (n + 7) / 8; i += stride) hints[i] = ~0u;
+    }
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) level[i] = BFS_UNREACHED;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         iter->value = 0u;

@@ -270,6 +270,49 @@ class EventProgram {
         if (hz::wave::ballot(pending) != 0 && hz::wave::leader()) set_flags(OVERFLOW_FLAG);
     }
 
+    // Queues up to K promises of one operation per active lane, those with
+    // want[k], with one atomic for all of them while the home segment has
+    // room.
+    template <typename TYPE, int K>
+    __device__ void async_each(int depth_delta, const Promise<TYPE> (&values)[K], const bool (&want)[K]) {
+        constexpr OpDisc D = Lookup<TYPE>::type::DISC;
+        static_assert(Lookup<TYPE>::type::CONTAINED, "operation is not part of this program's OpSet");
+        uint32_t at[K], total = 0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const uint64_t m = hz::wave::ballot(want[k]);
+            at[k] = total + hz::wave::rank(m);
+            total += hz::wave::popc(m);
+        }
+        if (total == 0u) return;
+        const unsigned int out = _grp_ctx.toggle ^ 1u;
+        const uint32_t cap = _dev_ctx.seg_capacity;
+        const uint32_t s = home_segment();
+        uint32_t base = 0;
+        if (hz::wave::leader()) base = hz::wave::atomic_add(&segment(D, s).out_count, total);
+        base = hz::wave::first(base);
+        bool left = false;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (want[k] && base + at[k] < cap) {
+                PromiseUnionType pu;
+                pu.template cast<TYPE>() = values[k];
+                uint32_t words[WORDS];
+                __builtin_memcpy(words, &pu, sizeof(PromiseUnionType));
+                const size_t i = (size_t)s * cap + base + at[k];
+#pragma unroll
+                for (uint32_t w = 0; w < WORDS; ++w) queue_row(out, D, w)[i] = words[w];
+            } else if (want[k]) {
+                left = true;
+            }
+        }
+        if (hz::wave::ballot(left) == 0ull) return;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (want[k] && base + at[k] >= cap) async_call_cast(depth_delta, values[k]);
+        }
+    }
+
     // Depth level of the promise being evaluated: a level-synchronous
     // program keeps no levels, so always 0.
     __device__ unsigned int depth() { return 0u; }

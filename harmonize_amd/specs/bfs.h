@@ -48,11 +48,26 @@ struct BfsJob {
 };
 
 struct BfsState {
+    static constexpr bool HINTS = false;
     const BfsJob* jobs;
     util::iter::AtomicIter<unsigned int>* job_iter;  // jobs still to start
     unsigned int job_count;
     unsigned int split;  // edge ranges longer than this are split
 };
+
+// The state of a search with level hints (BfsSpecT): the jobs' level arrays
+// lie one after another from level_base, and hints holds four bits per vertex
+// in the same order, an upper bound of its level up to 14, or BFS_NO_HINT.
+struct BfsHintState {
+    static constexpr bool HINTS = true;
+    const BfsJob* jobs;
+    util::iter::AtomicIter<unsigned int>* job_iter;
+    unsigned int job_count;
+    unsigned int split;
+    unsigned char* hints;
+    const int32_t* level_base;
+};
+constexpr int BFS_NO_HINT = 15;
 
 struct BfsVisit;
 struct BfsEdges;
@@ -66,8 +81,9 @@ struct BfsVisit {
     template <typename PROGRAM>
     __device__ static void eval(PROGRAM prog, unsigned int job, int vertex, int level) {
         const BfsJob j = prog.device.jobs[job];
+        const int begin = j.row_ptr[vertex], end = j.row_ptr[vertex + 1];  // on their way with the level
         if (hz_load(&j.level[vertex]) < level) return;
-        bfs_relax(prog, job, j, j.row_ptr[vertex], j.row_ptr[vertex + 1], level + 1);
+        bfs_relax(prog, job, j, begin, end, level + 1);
     }
 };
 
@@ -85,12 +101,24 @@ struct BfsEdges {
 #if defined(__HIP_DEVICE_COMPILE__)
 // One lane's edge range, as the wavefront shares it in LDS (32 bytes).
 struct BfsRange {
-    const int32_t* col;  // first column of the range
+    const int32_t* col;  // first column of the range, less its start
     int32_t* level;      // the job's level array
-    unsigned int start;  // exclusive prefix of the wavefront's range lengths
+    uint64_t vertex;     // the job's first vertex among all jobs' (level hints)
     unsigned int job;
     int next;            // level written to the range's targets
-    unsigned int pad;
+};
+
+// A pointer that was read back from LDS is taken for one into any memory,
+// which costs flat instructions (they occupy the LDS path too): these say
+// that it points to device memory.
+typedef const __attribute__((address_space(1))) int32_t* BfsColumn;
+typedef __attribute__((address_space(1))) int32_t* BfsLevel;
+
+// HZ_BFS_CHAINS edges of one lane, up to the read of their targets.
+struct BfsEdgeSet {
+    unsigned int owner[HZ_BFS_CHAINS];  // row of the range
+    int w[HZ_BFS_CHAINS];
+    bool has[HZ_BFS_CHAINS];
 };
 
 // Relaxes the edge ranges of all active lanes together: edge e of the
@@ -100,12 +128,24 @@ struct BfsRange {
 // [0, n) of its wavefront's LDS block are exactly the live ones), and the
 // prefix of range lengths comes from ballots over their bit slices, so
 // inactive lanes are never read.
+//
+// A round takes HZ_BFS_CHAINS edges per lane and waits for memory, not for
+// bandwidth: columns, then hints (or levels), then the atomics. The columns
+// of the next round are looked up and read while the hints of this one are
+// on their way, and the visits of a round are queued in one step
+// (async_each). The 64-graph batch (14..22 bits of vertices, 1.1e9 edges
+// looked at): EventProgram 19.4 ms with a look-up, a read and a queue append
+// after another, 16.7 by hints, 14.7 so; AsyncProgram 19.7 and 18.6.
 template <typename PROGRAM>
 __device__ inline void bfs_relax_wave(PROGRAM& prog, unsigned int job, const BfsJob& j, int begin, int end,
                                       int next) {
+    constexpr int CH = HZ_BFS_CHAINS;
+    constexpr bool HINTS = PROGRAM::DeviceState::HINTS;
     constexpr unsigned int WAVES = (unsigned int)(PROGRAM::WORK_GROUP_SIZE / 64);
     __shared__ BfsRange ranges[WAVES][64];
+    __shared__ unsigned int starts[WAVES][64];  // exclusive prefixes of the range lengths
     BfsRange* row = ranges[hz_block_thread() / 64u];
+    unsigned int* row_start = starts[hz_block_thread() / 64u];
     const uint64_t live = hz::wave::active();
     const unsigned int n = hz::wave::popc(live);
     const unsigned int me = hz::wave::rank(live);
@@ -116,46 +156,113 @@ __device__ inline void bfs_relax_wave(PROGRAM& prog, unsigned int job, const Bfs
         start += hz::wave::rank(m) << b;
         total += hz::wave::popc(m) << b;
     }
-    row[me] = BfsRange{j.col + begin, j.level, start, job, next, 0u};
+    uint64_t vertex = 0u;
+    if constexpr (HINTS) vertex = (uint64_t)(j.level - prog.device.level_base);
+    row[me] = BfsRange{j.col + begin - (long long)start, j.level, vertex, job, next};
+    row_start[me] = start;
+    for (unsigned int i = n + me; i < 64u; i += n) row_start[i] = ~0u;
     hz::wave::sync();
-    // HZ_BFS_CHAINS edges per lane per round keep that many memory chains in
-    // flight.
-    constexpr int CH = HZ_BFS_CHAINS;
-    for (unsigned int base = 0; base < total; base += (unsigned int)CH * n) {
-        int w[CH], seen[CH], before[CH];
-        const BfsRange* owner[CH];
-        bool has[CH];
+
+    auto take = [&](unsigned int base, BfsEdgeSet& s) {
+        unsigned int lo[CH];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) lo[k] = 0u;
+        // The last range starting at or before an edge holds it: ranges of
+        // length 0 share their successor's start.
+#pragma unroll
+        for (unsigned int step = 32u; step != 0u; step >>= 1) {
+            unsigned int at[CH];
+#pragma unroll
+            for (int k = 0; k < CH; ++k) at[k] = row_start[lo[k] + step];
+#pragma unroll
+            for (int k = 0; k < CH; ++k) lo[k] += at[k] <= base + (unsigned int)k * n + me ? step : 0u;
+        }
 #pragma unroll
         for (int k = 0; k < CH; ++k) {
             const unsigned int e = base + (unsigned int)k * n + me;
-            has[k] = e < total;
-            owner[k] = row;
-            w[k] = 0;
-            if (has[k]) {
-                // The last range starting at or before e holds it: ranges
-                // of length 0 share their successor's start.
-                unsigned int lo = 0u, hi = n - 1u;
-                while (lo < hi) {
-                    const unsigned int mid = (lo + hi + 1u) >> 1;
-                    if (row[mid].start <= e) lo = mid; else hi = mid - 1u;
+            s.owner[k] = lo[k];
+            s.has[k] = e < total;
+            s.w[k] = 0;
+            if (s.has[k]) s.w[k] = __builtin_nontemporal_load((BfsColumn)row[lo[k]].col + e);
+        }
+    };
+
+    BfsEdgeSet edges, ahead;
+    auto level_of = [&](int k) {
+        return __hip_atomic_load((BfsLevel)row[edges.owner[k]].level + edges.w[k], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+    };
+    take(0u, edges);
+    for (unsigned int base = 0; base < total; base += (unsigned int)CH * n) {
+        Promise<BfsVisit> visit[CH];
+        bool lowered[CH];
+        int seen[CH], before[CH];
+        uint64_t at[CH];
+        if constexpr (HINTS) {
+            // Level hints. Levels only fall, so any value a vertex's hint
+            // ever had bounds its level from above, however stale the copy
+            // that is read, and a target whose hint is at most `next` needs
+            // no look at its level. The hints of a graph take an eighth of
+            // its levels' bytes, so more of them are found in the XCD's L2:
+            // 57 % of all requests, where it was a third (fetched beyond the
+            // L2 58 to 34 GB).
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                at[k] = row[edges.owner[k]].vertex + (unsigned int)edges.w[k];
+                seen[k] = edges.has[k] ? (int)__hip_atomic_load(prog.device.hints + (at[k] >> 1), __ATOMIC_RELAXED,
+                                                                __HIP_MEMORY_SCOPE_WORKGROUP)
+                                       : 0;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                seen[k] = edges.has[k] ? level_of(k) : 0;
+            }
+        }
+        const unsigned int then = base + (unsigned int)CH * n;
+        if (then < total) take(then, ahead);
+        int byte[CH];
+        if constexpr (HINTS) {
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                const int nx = row[edges.owner[k]].next;
+                byte[k] = seen[k];
+                const int hint = byte[k] >> (4u * ((unsigned int)at[k] & 1u)) & 15;
+                edges.has[k] = edges.has[k] && (hint == BFS_NO_HINT || hint > nx);
+                // Beyond the hints' range the level itself says whether the
+                // atomic can lower it.
+                seen[k] = BFS_UNREACHED;
+                if (edges.has[k] && nx >= BFS_NO_HINT) seen[k] = level_of(k);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            const int nx = row[edges.owner[k]].next;
+            before[k] = edges.has[k] && seen[k] > nx ? __hip_atomic_fetch_min((BfsLevel)row[edges.owner[k]].level + edges.w[k], nx, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT) : nx;
+        }
+        if constexpr (HINTS) {
+            // The neighbour's half of the byte may be lost to another lane's
+            // write: it then says what it said before, which still holds.
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                const int nx = row[edges.owner[k]].next;
+                if (edges.has[k] && nx < BFS_NO_HINT) {
+                    const unsigned int shift = 4u * ((unsigned int)at[k] & 1u);
+                    __hip_atomic_store(prog.device.hints + (at[k] >> 1),
+                                       (unsigned char)((byte[k] & ~(15 << shift)) | nx << shift), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-                owner[k] = row + lo;
-                w[k] = owner[k]->col[e - owner[k]->start];
             }
         }
 #pragma unroll
-        for (int k = 0; k < CH; ++k) seen[k] = has[k] ? hz_load(&owner[k]->level[w[k]]) : 0;
-#pragma unroll
         for (int k = 0; k < CH; ++k) {
-            const int nx = owner[k]->next;
-            before[k] = has[k] && seen[k] > nx ? atomicMin(&owner[k]->level[w[k]], nx) : nx;
+            const int nx = row[edges.owner[k]].next;
+            lowered[k] = edges.has[k] && before[k] > nx;
+            visit[k] = Promise<BfsVisit>(row[edges.owner[k]].job, edges.w[k], nx);
         }
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            if (has[k] && before[k] > owner[k]->next) {
-                prog.template async_call_cast<BfsVisit>(1, Promise<BfsVisit>(owner[k]->job, w[k], owner[k]->next));
-            }
-        }
+        prog.async_each(1, visit, lowered);
+        edges = ahead;
     }
     hz::wave::sync();
 }
@@ -206,10 +313,11 @@ __device__ inline void bfs_relax(PROGRAM& prog, unsigned int job, const BfsJob& 
 
 // GROUPS: wavefront groups per workgroup (the launch's work-group size / 64);
 // STASH: LDS links per group (fewer links, more resident wavefronts).
-template <unsigned int GROUPS, unsigned int STASH = 16>
+// HINTS: levels are looked up through hints first (BfsHintState).
+template <unsigned int GROUPS, unsigned int STASH = 16, bool HINTS = false>
 struct BfsSpecT {
     typedef OpUnion<BfsVisit, BfsEdges> OpSet;
-    typedef BfsState DeviceState;
+    typedef typename std::conditional<HINTS, BfsHintState, BfsState>::type DeviceState;
 
     static const size_t STASH_SIZE = STASH;
     static const size_t FRAME_SIZE = 8;
@@ -217,8 +325,8 @@ struct BfsSpecT {
     static const size_t GROUPS_PER_BLOCK = GROUPS;
     // A search grows from one vertex per graph: hand links to idle groups.
     static const size_t SHARE_WORK = 1;
-    // Besides its promise a visit reads the graph, which does not change, and
-    // levels at the coherence point.
+    // Besides its promise a visit reads the graph, which does not change,
+    // levels at the coherence point and hints, which may be stale.
     static const size_t LINK_ACQUIRE = 0;
     // Run the links that filled first first, closer to level order: fewer
     // vertices are visited again at a lower level (77 M -> 69 M promises at
