@@ -278,6 +278,9 @@ class AsyncProgram {
     static_assert(GROUPS_PER_BLOCK >= 1 && GROUPS_PER_BLOCK <= 16, "GROUPS_PER_BLOCK must be in [1, 16]");
     static const size_t WORK_GROUP_SIZE = 64 * GROUPS_PER_BLOCK;
     static constexpr bool SHARE_WORK = hz::spec::SHARE_WORKOr<PROGRAM_SPEC, 0>::value != 0;
+    // Whether resolving a unit future publishes all that its promise wrote,
+    // or the returned value only (see hz::resolve_value).
+    static constexpr bool RETURN_RELEASE = hz::spec::RETURN_RELEASEOr<PROGRAM_SPEC, 1>::value != 0;
     // Whether a group that takes a link off a queue acquires what its
     // promises' makers have released besides the promises themselves. An
     // acquire empties the caches that the XCD's other wavefronts read through.
@@ -958,16 +961,7 @@ class AsyncProgram {
         return best_link;
     }
 
-    // Waits until this wavefront's earlier memory operations have completed:
-    // write-through stores are then at the device's coherence point, so a
-    // later relaxed store that publishes them needs no release fence (which
-    // would write back the XCD's whole L2). The signal fences keep the
-    // compiler from moving memory operations across the wait.
-    __device__ static HZ_INLINE void stores_done() {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    }
+    __device__ static HZ_INLINE void stores_done() { hz::wave::stores_done(); }
 
     // Moves stash link L to the arena and queues it. Cooperative over the
     // active lanes (all 64 in the scheduler loop, a subset inside an async

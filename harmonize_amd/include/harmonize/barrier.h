@@ -178,6 +178,15 @@ struct UnitBarrier {
         add_semaphore(program, 0u - delta);
     }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+    // Counts a fulfilment whose value is at the device's coherence point and
+    // is read there: nothing is released, nothing acquired.
+    template <typename PROGRAM>
+    __device__ HZ_INLINE void count_returned(PROGRAM program) {
+        if (hz::wave::atomic_add(&semaphore.sem, ~0u) == 1u && promise.disc != NO_PROMISE) program.async_call(promise);
+    }
+#endif
+
    private:
     template <typename PROGRAM>
     __device__ HZ_INLINE void fire(PROGRAM program) {

@@ -491,6 +491,7 @@ class EventProgram {
 
     // Promises cannot be held on a RemappingBarrier (see barrier_await).
     static constexpr bool REMAPPING_AWAIT = false;
+    static constexpr bool RETURN_RELEASE = hz::spec::RETURN_RELEASEOr<PROGRAM_SPEC, 1>::value != 0;
     // Records a misuse of the future API; complete() reports it.
     __device__ void usage_error() { set_flags(USAGE_FLAG); }
 

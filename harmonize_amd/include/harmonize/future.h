@@ -208,8 +208,35 @@ __device__ __host__ HZ_INLINE void forward_promise(PROGRAM program, ENUM pe, Ret
 
 }  // namespace detail
 
+// A resolution orders everything its promise wrote before the promise that
+// waits for it: a release, which on gfx950 writes back the XCD's whole L2, and
+// on the last fulfilment an acquire. A specification whose value-returning
+// operations hand over nothing but the returned value, and whose operations
+// read such values with hz_load, says so (RETURN_RELEASE = 0): a unit
+// future's value is then written through and waited for instead. (The futures
+// demo, 2^20 chains and as many joins: 2.4 million evaluations in 13.3 ms,
+// two fifths of them with a write-back; 4.7 ms without.)
 template <typename PROGRAM, typename TYPE>
 __device__ __host__ HZ_INLINE void resolve_value(PROGRAM program, ReturnAdr<TYPE> adr, const TYPE& value) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (!PROGRAM::RETURN_RELEASE && (sizeof(TYPE) == 4 || sizeof(TYPE) == 8) &&
+                  alignof(TYPE) == sizeof(TYPE)) {
+        // The store and the look at the kind of barrier are one wait.
+        using Bits = typename std::conditional<sizeof(TYPE) == 8, unsigned long long, unsigned int>::type;
+        Bits bits;
+        __builtin_memcpy(&bits, &value, sizeof(TYPE));
+        if (adr.dest != nullptr) hz::wave::atomic_store((Bits*)adr.dest, bits);
+        if (adr.base == nullptr) return;
+        const unsigned int tag = adr.base->tag;
+        hz::wave::stores_done();
+        if (tag == UNIT_BARRIER_TAG) {
+            reinterpret_cast<UnitBarrier<typename PROGRAM::OpSet>*>(adr.base)->count_returned(program);
+        } else {
+            fulfill(program, adr.base);
+        }
+        return;
+    }
+#endif
     if (adr.dest != nullptr) *adr.dest = value;
     fulfill(program, adr.base);
 }

@@ -53,6 +53,7 @@ HZ_CONST_OR(GROUPS_PER_BLOCK)
 // none (for work that grows from few seeds). Not a reference constant.
 HZ_CONST_OR(SHARE_WORK)
 HZ_CONST_OR(LINK_ACQUIRE)
+HZ_CONST_OR(RETURN_RELEASE)
 // Nonzero: a group runs its ready links oldest first (the order in which
 // they filled), rather than by stash position. Work whose later promises can
 // supersede earlier ones (a BFS level lowered again) wastes less. Not a

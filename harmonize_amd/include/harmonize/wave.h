@@ -95,6 +95,17 @@ __device__ HZ_INLINE void fence_acq_rel() { __builtin_amdgcn_fence(__ATOMIC_ACQ_
 __device__ HZ_INLINE void fence_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
 __device__ HZ_INLINE void fence_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
+// Waits until this wavefront's earlier memory operations have completed:
+// write-through stores are then at the device's coherence point, so a later
+// relaxed store or atomic that publishes them needs no release fence (which
+// would write back the XCD's whole L2). The signal fences keep the compiler
+// from moving memory operations across the wait.
+__device__ HZ_INLINE void stores_done() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 // Fetch-and-add where every active lane asks for `amount`: one atomic per
 // wavefront, each lane receiving the start of its own disjoint range in lane
 // order. Lanes asking for different amounts fall back to one atomic each.
