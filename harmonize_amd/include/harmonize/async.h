@@ -2446,9 +2446,18 @@ class AsyncProgram {
 
     // Any-lane arena allocation (the wave's spare cache is single-lane).
     __device__ HZ_INLINE unsigned int arena_alloc_any() {
-        unsigned int id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
-        if (id != hz::LINK_NONE) return id;
-        if (hz::wave::atomic_load(&_dev_ctx.status->claim) < _dev_ctx.links) {
+        // The two counts are looked at through the caches first: they are
+        // one word each for the device, and what a stale copy hides only
+        // costs a link its reuse.
+        auto cached = [](const auto* p) {
+            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        unsigned int id = hz::LINK_NONE;
+        if (cached(&_dev_ctx.free_queue->count) > 0) {
+            id = queue_pop(_dev_ctx.free_queue, _dev_ctx.free_slots, false);
+            if (id != hz::LINK_NONE) return id;
+        }
+        if (cached(&_dev_ctx.status->claim) < _dev_ctx.links) {
             unsigned int claim = hz::wave::atomic_add(&_dev_ctx.status->claim, 1u);
             if (claim < _dev_ctx.links) return claim;
         }

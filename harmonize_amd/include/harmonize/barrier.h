@@ -121,7 +121,7 @@ struct RemappingBarrier {
     template <typename PROGRAM>
     __device__ HZ_INLINE void add_semaphore(PROGRAM program, unsigned int delta) {
         hz_fence_release();
-        unsigned int before = atomicAdd(&semaphore.sem, delta);
+        unsigned int before = hz_add_semaphore(&semaphore.sem, delta);
         if (before + delta == 0u) {
             hz_fence_acquire();
             program.barrier_release(*this);
@@ -169,7 +169,7 @@ struct UnitBarrier {
     template <typename PROGRAM>
     __device__ HZ_INLINE void add_semaphore(PROGRAM program, unsigned int delta) {
         hz_fence_release();
-        unsigned int old_val = atomicAdd(&semaphore.sem, delta);
+        unsigned int old_val = hz_add_semaphore(&semaphore.sem, delta);
         if ((old_val + delta) == 0u && old_val != 0u) fire(program);
     }
 

@@ -137,7 +137,20 @@ __device__ HZ_INLINE unsigned int hz_block_thread() { return threadIdx.x; }
 __device__ HZ_INLINE unsigned int hz_block_threads() { return blockDim.x; }
 
 // Platform hooks used by the portable barrier layer: device-wide release and
-// acquire ordering around semaphore updates.
+// acquire ordering around semaphore updates, and the update itself, one
+// atomic where every active lane names the same semaphore and amount (each
+// lane's result is what its own atomic in lane order would return).
+__device__ HZ_INLINE unsigned int hz_add_semaphore(unsigned int* sem, unsigned int delta) {
+    const uint64_t act = hz::wave::active();
+    const uint64_t addr = (uint64_t)(uintptr_t)sem;
+    if (hz::wave::ballot(addr == hz::wave::first(addr) && delta == hz::wave::first(delta)) == act) {
+        const uint32_t r = hz::wave::rank(act);
+        unsigned int before = 0u;
+        if (r == 0u) before = hz::wave::atomic_add(sem, delta * hz::wave::popc(act));
+        return hz::wave::first(before) + r * delta;
+    }
+    return hz::wave::atomic_add(sem, delta);
+}
 __device__ HZ_INLINE void hz_fence_release() { hz::wave::fence_release(); }
 __device__ HZ_INLINE void hz_fence_acquire() { hz::wave::fence_acquire(); }
 

@@ -34,6 +34,9 @@ inline void __syncthreads() {}
 
 // Ordering around barrier semaphore updates (the atomics below are
 // sequentially consistent already; the fences keep plain stores ordered).
+inline unsigned int hz_add_semaphore(unsigned int* sem, unsigned int delta) {
+    return __atomic_fetch_add(sem, delta, __ATOMIC_SEQ_CST);
+}
 inline void hz_fence_release() { __atomic_thread_fence(__ATOMIC_RELEASE); }
 inline void hz_fence_acquire() { __atomic_thread_fence(__ATOMIC_ACQUIRE); }
 
