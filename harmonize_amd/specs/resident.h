@@ -34,6 +34,7 @@
 // finished job can later overwrite memory the host has reused.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 #include "collatz.h"
@@ -90,9 +91,9 @@ struct ResidentDoorbell {
 };
 
 // One installed job (device memory).
-struct ResidentJob {
+struct alignas(8) ResidentJob {
     unsigned int next;         // items claimed; CLOSED while the entry takes no claims
-    unsigned int limit;        // items
+    unsigned int limit;        // items (claims read both as one 64-bit word)
     unsigned int entry;        // ring sequence number of its descriptor
     unsigned int pad;
     unsigned long long seed;
@@ -153,6 +154,8 @@ struct ResidentClaim {
     unsigned int pend_job;  // job of the pending ends
     unsigned int pend;      // ends not yet added to the `ended` counters
     unsigned int held;
+    unsigned int base;      // the claimed job's item space and seed
+    unsigned long long seed;
     unsigned long long poll_seen;
 };
 
@@ -251,23 +254,18 @@ __device__ HZ_INLINE void flush_ends(const ResidentState& s, ResidentClaim& t) {
     t.pend = 0u;
 }
 
-// State of an installed job (the whole wavefront calls it with the same
-// job): items left to claim, every item claimed, or finished (every item and
-// everything created from them has ended). The `ended` scan completes before
-// the `created` scan is issued.
-constexpr unsigned int JOB_OPEN = 0u, JOB_CLAIMED = 1u, JOB_FINISHED = 2u;
-
-__device__ HZ_INLINE unsigned int job_state(const ResidentState& s, unsigned int job) {
-    ResidentJob& J = s.core->jobs[job];
-    const unsigned int limit = hz::wave::first(ld(&J.limit));
-    const unsigned int next = hz::wave::first(ld(&J.next));
-    if (next < limit) return JOB_OPEN;
+// Whether a job whose `limit` items are all claimed has finished: every item
+// and everything created from them has ended (the whole wavefront calls it
+// with the same job). The `ended` scan completes before the `created` scan is
+// issued.
+__device__ HZ_INLINE bool job_ended(const ResidentState& s, unsigned int job, unsigned int limit) {
     const uint32_t lane = hz::wave::lane();
     unsigned int e = lane < STRIPES ? ld(counter(s, job, 0u, lane)) : 0u;
     e = hz::wave::first(wave_sum(e));
+    stores_done();
     unsigned int c = lane < STRIPES ? ld(counter(s, job, 1u, lane)) : 0u;
     c = hz::wave::first(wave_sum(c));
-    return e == limit + c ? JOB_FINISHED : JOB_CLAIMED;
+    return e == limit + c;
 }
 
 // Installs ring entry k into its job table entry (the whole wavefront, under
@@ -306,21 +304,22 @@ __device__ HZ_INLINE bool install(const ResidentState& s, unsigned int k, unsign
     KIND::install(s, word_at(4));
     // Claims that see the job open see its fields and zeroed counters.
     stores_done();
+    // Claim order: append, or insert before the first larger job (the list
+    // is in order of size then).
+    const unsigned int listed = lane < n ? ld(&core->active[lane]) : JOBS;
+    const unsigned int listed_size = lane < n ? ld(&core->active_size[lane]) : 0u;
+    unsigned int at = n;
+    if (s.policy == SMALLEST_FIRST) at = hz::wave::popc(hz::wave::ballot(lane < n && listed_size <= size));
     if (lane == 0) {
         st(&J.next, 0u);
         __hip_atomic_fetch_or(&core->open_jobs, 1ull << job, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // Claim order: append, or insert before the first larger job.
-        unsigned int at = n;
-        if (s.policy == SMALLEST_FIRST) {
-            while (at > 0 && ld(&core->active_size[at - 1]) > size) --at;
-        }
-        for (unsigned int i = n; i > at; --i) {
-            st(&core->active[i], ld(&core->active[i - 1]));
-            st(&core->active_size[i], ld(&core->active_size[i - 1]));
-        }
         st(&core->active[at], job);
         st(&core->active_size[at], size);
         st(&core->installs, ld(&core->installs) + 1u);
+    }
+    if (lane >= at && lane < n) {
+        st(&core->active[lane + 1u], listed);
+        st(&core->active_size[lane + 1u], listed_size);
     }
     stores_done();
     if (lane == 0) st(&core->active_count, n + 1u);
@@ -365,29 +364,45 @@ __device__ HZ_INLINE void poll(const ResidentState& s, ResidentClaim& t) {
     unsigned int n = hz::wave::first(ld(&core->active_count));
     if (n > JOBS) n = JOBS;
     const unsigned long long open = hz::wave::first((uint64_t)ld(&core->open_jobs));
-    for (unsigned int i = 0; i < n;) {
-        const unsigned int job = hz::wave::first(ld(&core->active[i]));
-        const unsigned int state = job < JOBS ? job_state(s, job) : JOB_OPEN;
-        if (state != JOB_OPEN && (open >> job & 1ull) && lane == 0) {
-            __hip_atomic_fetch_and(&core->open_jobs, ~(1ull << job), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // A list place per lane. (Read, tested and moved up place by place, a
+    // pass over 48 jobs cost some 5 microseconds for each and a job that left
+    // the list up to 100: a job's end was noticed late, and 48 jobs that end
+    // together took 2 ms of the batch's 11.)
+    const bool there = lane < n;
+    const unsigned int job = there ? ld(&core->active[lane]) : JOBS;
+    const unsigned int size = there ? ld(&core->active_size[lane]) : 0u;
+    unsigned int limit = 0u;
+    bool all_claimed = false, finished = false;
+    if (job < JOBS) {
+        const unsigned long long both = ld((const unsigned long long*)&core->jobs[job]);
+        limit = (unsigned int)(both >> 32);
+        all_claimed = (unsigned int)both >= limit;
+    }
+    for (uint64_t m = hz::wave::ballot(all_claimed); m != 0ull; m &= m - 1ull) {
+        const uint32_t i = (uint32_t)__builtin_ctzll(m);
+        const bool ended = job_ended(s, hz::wave::read_lane(job, i), hz::wave::read_lane(limit, i));
+        if (lane == i) finished = ended;
+    }
+    if (all_claimed && (open >> job & 1ull)) {
+        __hip_atomic_fetch_and(&core->open_jobs, ~(1ull << job), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const uint64_t done = hz::wave::ballot(finished);
+    if (done != 0ull) {
+        const uint64_t keep = hz::wave::ballot(there && !finished);
+        const unsigned int entry = finished ? ld(&core->jobs[job].entry) : 0u;
+        if (there && !finished) {
+            const unsigned int at = hz::wave::rank(keep);
+            st(&core->active[at], job);
+            st(&core->active_size[at], size);
         }
-        if (state != JOB_FINISHED) {
-            ++i;
-            continue;
-        }
+        n = hz::wave::popc(keep);
         if (lane == 0) {
-            for (unsigned int m = i; m + 1u < n; ++m) {
-                st(&core->active[m], ld(&core->active[m + 1u]));
-                st(&core->active_size[m], ld(&core->active_size[m + 1u]));
-            }
-            st(&core->active_count, n - 1u);
-            st(&core->completions, ld(&core->completions) + 1u);
-            const unsigned int entry = ld(&core->jobs[job].entry);
-            stores_done();
-            sys_st(&s.bell->done[entry % RING], entry + 1u);
+            st(&core->active_count, n);
+            st(&core->completions, ld(&core->completions) + hz::wave::popc(done));
         }
+        stores_done();
+        if (finished) sys_st(&s.bell->done[entry % RING], entry + 1u);
         hz::wave::sync();
-        n -= 1u;
     }
 
     // New entries, while the table has room.
@@ -435,44 +450,75 @@ __device__ HZ_INLINE bool claim(const ResidentState& s, ResidentClaim& t, bool& 
     if (need == 0ull) return true;
     ResidentCore* core = s.core;
     const uint32_t lane = hz::wave::lane();
+    // Every group that claims reads the same words, and one line passes a
+    // load every 30 ns: the core's first words are one load, a word per
+    // lane, and a job's claim counter and limit another.
     const unsigned int slot = ld(&core->active[lane]);
-    const unsigned int n = hz::wave::first(ld(&core->active_count));
-    const unsigned long long open = hz::wave::first((uint64_t)ld(&core->open_jobs));
-    stopping = hz::wave::first(ld(&core->stopping)) != 0u;
+    const unsigned int head = ld((const unsigned int*)core + (lane & 7u));
+    auto head_at = [&](size_t byte) { return hz::wave::read_lane(head, (uint32_t)(byte / 4u)); };
+    const unsigned int n = head_at(offsetof(ResidentCore, active_count));
+    const unsigned long long open = head_at(offsetof(ResidentCore, open_jobs)) |
+                                    (unsigned long long)head_at(offsetof(ResidentCore, open_jobs) + 4) << 32;
+    stopping = head_at(offsetof(ResidentCore, stopping)) != 0u;
     if (stopping || open == 0ull) return false;
     const bool listed = lane < n && slot < JOBS && (open >> slot & 1ull);
     unsigned int seen = 0u, limit = 0u;
     if (listed) {
-        seen = ld(&core->jobs[slot].next);
-        limit = ld(&core->jobs[slot].limit);
+        const unsigned long long both = ld((const unsigned long long*)&core->jobs[slot]);
+        seen = (unsigned int)both;
+        limit = (unsigned int)(both >> 32);
     }
     uint64_t avail = hz::wave::ballot(listed && seen < limit);
     const unsigned int want_lanes = hz::wave::popc(need);
+    // Items left in all open jobs: in order of admission, a wavefront that
+    // takes more of one job leaves the others to the rest.
+    unsigned int all_left = 0u;
+    if constexpr (KIND::SHARES_OF_ALL) {
+        if (s.policy == BY_ADMISSION) {
+            const unsigned int mine = listed && seen < limit ? limit - seen : 0u;
+            all_left = wave_sum(mine < 0x2000000u ? mine : 0x2000000u);
+        }
+    }
     while (avail != 0ull) {
         const uint32_t lead = (uint32_t)__builtin_ctzll(avail);
         avail &= avail - 1ull;
         unsigned int base = 0u, got = 0u, per = 1u;
         if (lane == lead) {
-            per = KIND::per_lane(limit - seen, gridDim.x * blockDim.x);
+            const unsigned int left = limit - seen;
+            per = KIND::per_lane(left > all_left ? left : all_left, gridDim.x * blockDim.x);
+            if (KIND::SHARES_OF_ALL && per > 1u && (uint64_t)per * want_lanes > left) {
+                per = (left + want_lanes - 1u) / want_lanes;
+            }
             ResidentJob& J = core->jobs[slot];
             const unsigned int want = want_lanes * per;
             const unsigned int old = __hip_atomic_fetch_add(&J.next, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // The job entry may have been replaced since it was read: the
-            // limit that counts is the one read after the claim.
-            const unsigned int lim = ld(&J.limit);
+            // limit that counts is the one read after the claim, below.
             base = old;
-            got = old < lim ? (lim - old < want ? lim - old : want) : 0u;
+            got = want;
         }
-        got = hz::wave::read_lane(got, lead);
-        if (got == 0u) continue;
+        const unsigned int job = hz::wave::read_lane(slot, lead);
         base = hz::wave::read_lane(base, lead);
         per = hz::wave::read_lane(per, lead);
-        const unsigned int job = hz::wave::read_lane(slot, lead);
+        got = hz::wave::read_lane(got, lead);
+        stores_done();
+        // The entry again, in one load, a word per lane: it stays while items
+        // claimed from it are left.
+        const unsigned int word = ld((const unsigned int*)&core->jobs[job] + (lane & 7u));
+        auto word_of = [&](size_t byte) { return hz::wave::read_lane(word, (uint32_t)(byte / 4u)); };
+        const unsigned int lim = word_of(offsetof(ResidentJob, limit));
+        got = base < lim ? (lim - base < got ? lim - base : got) : 0u;
+        if (got == 0u) continue;
         claimed = job;
         bulk = per > 1u;
         if (t.next >= t.end) {
             const unsigned int r = hz::wave::rank(need) * per;
             t.job = job;
+            if constexpr (KIND::CLAIMS_SEED) {
+                t.seed = word_of(offsetof(ResidentJob, seed)) |
+                         (unsigned long long)word_of(offsetof(ResidentJob, seed) + 4) << 32;
+                t.base = word_of(offsetof(ResidentJob, base));
+            }
             t.next = base + (r < got ? r : got);
             t.end = base + (r + per < got ? r + per : got);
         }
@@ -512,6 +558,8 @@ struct ResidentSpecT {
         prog.thread.pend_job = NO_JOB;
         prog.thread.pend = 0u;
         prog.thread.held = NO_JOB;
+        prog.thread.base = 0u;
+        prog.thread.seed = 0ull;
         prog.thread.poll_seen = 0ull;
         KIND::init_group(prog);
     }
@@ -609,6 +657,8 @@ struct RCollatzOdd {
 };
 
 struct ResidentCollatzKind {
+    static constexpr bool CLAIMS_SEED = true;
+    static constexpr bool SHARES_OF_ALL = true;
     typedef OpUnion<RCollatzEven, RCollatzOdd> OpSet;
     static const size_t STASH_SIZE = 7;
     static const size_t CHAIN_PASSES = HZ_COLLATZ_PASSES;
@@ -633,9 +683,8 @@ struct ResidentCollatzKind {
 
     template <typename PROGRAM>
     __device__ static HZ_INLINE void launch(PROGRAM& prog, unsigned int job, unsigned int index) {
-        ResidentJob& J = prog.device.core->jobs[job];
-        const unsigned long long seed = hz::resident::ld(&J.seed);
-        const unsigned int item = hz::resident::ld(&J.base) + index;
+        const unsigned long long seed = prog.thread.seed;
+        const unsigned int item = prog.thread.base + index;
         const unsigned long long modulus = (1ull << prog.device.bits) - 1ull;
         hz::philox::Ctr r = hz::philox::philox4x32_10(index, 0u, 0u, 0u, (uint32_t)seed, (uint32_t)(seed >> 32));
         const unsigned long long start = ((((unsigned long long)r.v[1] << 32) | r.v[0]) % modulus) + 1ull;
@@ -763,6 +812,8 @@ struct RPhotonStep {
 };
 
 struct ResidentPhotonKind {
+    static constexpr bool SHARES_OF_ALL = false;
+    static constexpr bool CLAIMS_SEED = false;  // launches read them with the job's tally
     typedef OpUnion<RPhotonStep> OpSet;
     static const size_t STASH_SIZE = HZ_PHOTON_STASH;
     static const size_t CHAIN_PASSES = 1;
