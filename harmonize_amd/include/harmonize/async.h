@@ -84,7 +84,7 @@ struct AsyncStatus {
     // barrier awaits into a barrier link. Every promise written is evaluated
     // exactly once, so appended = promises + those still queued or held.
     unsigned long long int appended;
-    // Promises run straight from registers by link forwarding (they are
+    // Promises run in the pass that queued them, from registers (they are
     // counted in `appended` and `promises` but never pass through a stash).
     unsigned long long int forwarded;
     // Shader-clock cycles per scheduler phase, summed over groups; filled only

@@ -67,13 +67,14 @@ struct BarrierDemoSpec {
     static const size_t POOL_SIZE = 8;
 
     // The source iterator and the counter are one word each for the whole
-    // device, which passes an atomic or a load every 30 ns: 2^22 ids claimed
-    // a wavefront at a time, with every evaluation counted as it ran, took
-    // 3.4 ms without a dependent and 11.2 with 2^21 of them on 64 barriers.
-    // Ids are claimed up to 8 per lane, and each thread counts for itself
-    // until the group leaves: 1.0 and 9.7 ms. (Up to 16 or 32 per lane leave
-    // the dependents, which come first, to half of the groups: 10.6.)
-    static const unsigned int CLAIM = 8;
+    // device, which passes an atomic or a load every 30 ns. Each thread
+    // counts for itself until the group leaves, and a claim is one load and
+    // one atomic: 2^21 awaits and as many ids without take 10.6 ms on 64
+    // barriers and 6.9 on 1,024 (11.7 and 7.6 with every evaluation counted
+    // as it ran). More ids per claim are faster for few and for very many
+    // barriers (8: 9.5 ms at 64, 5.6 at 8,192) and slower between them (14.8
+    // at 256 and 512, against 7.5): wavefronts then await in step.
+    static const unsigned int CLAIM = 1;
 
     template <typename PROGRAM>
     __device__ static void initialize(PROGRAM prog) {
