@@ -60,7 +60,7 @@ def algorithmic_bytes(promises: int, starts: int) -> int:
 # reads for a 1 GiB device-to-device copy (`bench.py --leg copy`): FETCH_SIZE
 # reads 512 MiB for the copy's 1 GiB of reads (factor 2.0) and WRITE_SIZE
 # reads 1 GiB for its 1 GiB of writes (factor 1.0).
-TRAFFIC_KIB = {"fetch": 1011086.5, "write": 2198988.1}
+TRAFFIC_KIB = {"fetch": 265766.0, "write": 266571.0}
 TRAFFIC_FACTOR = {"fetch": 2.0, "write": 1.0}
 
 
@@ -72,7 +72,7 @@ def measured_traffic_bytes() -> int:
 # `rocprofv3 --pmc SQ_INSTS_SALU SQ_INSTS_VALU SQ_INSTS_LDS SQ_INSTS_BRANCH
 # SQ_WAVES SQ_BUSY_CYCLES GRBM_GUI_ACTIVE GRBM_COUNT` pass over
 # `bench.py --leg collatz_async` (totals over all wavefronts of the dispatch).
-ISSUE_COUNTS = {"salu": 2.4486e10, "valu": 1.8018e10, "lds": 4.1635e9, "branch": 8.7764e9}
+ISSUE_COUNTS = {"salu": 2.82706e9, "valu": 4.62506e9, "lds": 5.76215e7, "branch": 6.56824e8}
 CLOCK_GHZ = 2.4  # MI355X peak engine clock
 LDS_BYTES_PER_CLOCK_PER_CU = 128
 
@@ -562,10 +562,12 @@ def main() -> int:
     per_launch_ms = kernel_ms / max(1, launches)
     per_launch_s = per_launch_ms * 1e-3
     cus = facts["compute_units"]
-    # The bound the headline kernel reaches: scalar instruction issue. A CU's
-    # four SIMDs share one scalar unit that issues at most one instruction per
-    # clock, so the chip's peak is CUs x clock.
-    salu_peak = cus * CLOCK_GHZ  # G SALU instructions/s
+    # The bound the headline kernel reaches: vector instruction issue. A wave64
+    # vector instruction occupies its SIMD for four clocks, so a CU's four
+    # SIMDs issue one per clock; so does the scalar unit they share, whose
+    # rate is reported beside it.
+    issue_peak = cus * CLOCK_GHZ  # G instructions/s, vector or scalar
+    valu_achieved = ISSUE_COUNTS["valu"] / max(1, launches) / per_launch_s / 1e9
     salu_achieved = ISSUE_COUNTS["salu"] / max(1, launches) / per_launch_s / 1e9
     # Beside it: the LDS bytes the stash moves (each promise that passes
     # through it is written into a link and read back out, 2 x 16 B; where
@@ -605,16 +607,18 @@ def main() -> int:
             "compute_units": facts["compute_units"],
         },
         "roofline": {
-            "bound": "salu",
-            "achieved": salu_achieved,
-            "peak": salu_peak,
-            "unit": "G SALU instructions/s",
-            "frac": salu_achieved / salu_peak,
+            "bound": "valu",
+            "achieved": valu_achieved,
+            "peak": issue_peak,
+            "unit": "G wave64 VALU instructions/s",
+            "frac": valu_achieved / issue_peak,
+            "salu": {"achieved": salu_achieved, "peak": issue_peak, "unit": "G SALU instructions/s",
+                     "frac": salu_achieved / issue_peak},
             "traffic": measured_traffic_bytes(),
             "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0)",
             "kernel": "_hz_exec_kernel<AsyncProgram<CollatzSpec>>",
             "kernel_ms": per_launch_ms,
-            "peak_model": f"one scalar instruction per CU per clock: {cus} CUs x {CLOCK_GHZ} GHz",
+            "peak_model": f"one wave64 vector instruction per CU per clock: {cus} CUs x {CLOCK_GHZ} GHz",
             "counts_per_launch": {k: v / max(1, launches) for k, v in ISSUE_COUNTS.items()},
             "counters": "profiles/collatz_async_issue_counters.md",
             "lds": {"achieved": lds_achieved, "peak": lds_peak, "unit": "GB/s", "frac": lds_achieved / lds_peak,
