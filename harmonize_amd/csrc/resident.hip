@@ -365,7 +365,7 @@ extern "C" int hz_resident_create(const hz_resident_config* config, hz_resident*
         {
             auto host = std::make_unique<ResidentCore>();
             std::memset(host.get(), 0, sizeof(ResidentCore));
-            for (unsigned int i = 0; i < R::JOBS; ++i) host->jobs[i].next = R::CLOSED;
+            for (unsigned int i = 0; i < R::JOBS; ++i) host->jobs[i].claims = R::claim_word(R::CLOSED, 0u);
             check(hipMemcpy(r->core, host.get(), sizeof(ResidentCore), hipMemcpyHostToDevice), "hipMemcpy(core)");
         }
         check(hipMemset(r->counters, 0, sizeof(unsigned int) * R::COUNTER_WORDS), "hipMemset(counters)");

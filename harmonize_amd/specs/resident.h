@@ -19,8 +19,9 @@
 // it.
 //
 // Job accounting, with no same-address hot spot:
-//  - items are claimed from the job's counter `next` (one atomic per
-//    wavefront claim); once `next` reaches `limit` every item has a claimant;
+//  - items are claimed from the job's claim word (claim_word.h), its counter
+//    and its limit in one (one atomic per wavefront claim); once the counter
+//    reaches the limit every item has a claimant;
 //  - whatever ends (a Collatz chain writing its step count) adds 1 to one of
 //    STRIPES `ended` counters after its own outputs have reached memory;
 //    entities created beyond the items (none for Collatz) would add to the
@@ -37,6 +38,7 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "claim_word.h"
 #include "collatz.h"
 #include "philox.h"
 #include "photon.h"
@@ -48,7 +50,6 @@ constexpr unsigned int JOBS = 64;           // job table entries
 constexpr unsigned int STRIPES = 16;        // accounting counters per job and kind
 constexpr unsigned int STRIPE_WORDS = 32;   // 128 bytes between counters
 constexpr unsigned int RING = 256;          // doorbell entries (a power of two)
-constexpr unsigned int CLOSED = 0x80000000u;
 constexpr unsigned int NO_JOB = 0xFFFFFFFFu;
 constexpr unsigned int COUNTER_WORDS = JOBS * 2u * STRIPES * STRIPE_WORDS;
 // Groups that take part in housekeeping (the first POLLERS of the launch,
@@ -91,9 +92,8 @@ struct ResidentDoorbell {
 };
 
 // One installed job (device memory).
-struct alignas(8) ResidentJob {
-    unsigned int next;         // items claimed; CLOSED while the entry takes no claims
-    unsigned int limit;        // items (claims read both as one 64-bit word)
+struct ResidentJob {
+    unsigned long long claims; // claim word: items claimed, or CLOSED (low half), and items in all
     unsigned int entry;        // ring sequence number of its descriptor
     unsigned int pad;
     unsigned long long seed;
@@ -196,6 +196,17 @@ __device__ HZ_INLINE void sys_st(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The claim words' memory (claim_word.h); stores come from the first lane.
+struct ClaimMemory {
+    __device__ HZ_INLINE unsigned long long add(unsigned long long* p, unsigned long long v) {
+        return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ HZ_INLINE void store(unsigned long long* p, unsigned long long v) {
+        if (hz::wave::lane() == 0) st(p, v);
+    }
+    __device__ HZ_INLINE void wait() { stores_done(); }
+};
+
 // Outputs are stored the same way: written through to memory.
 template <typename T>
 __device__ HZ_INLINE void store_out(T* p, T v) {
@@ -289,21 +300,20 @@ __device__ HZ_INLINE bool install(const ResidentState& s, unsigned int k, unsign
     }
     ResidentJob& J = core->jobs[job];
     const unsigned int size = word_at(1);
-    if (lane == 0) st(&J.next, CLOSED);
-    stores_done();
-    if (lane < STRIPES) {
-        st(counter(s, job, 0u, lane), 0u);
-        st(counter(s, job, 1u, lane), 0u);
-    }
-    if (lane == 0) {
-        st(&J.limit, size);
-        st(&J.entry, k);
-        st(&J.seed, pair_at(2));
-        st(&J.base, word_at(4));
-    }
-    KIND::install(s, word_at(4));
     // Claims that see the job open see its fields and zeroed counters.
-    stores_done();
+    ClaimMemory memory;
+    replace_job(memory, &J.claims, size, [&] {
+        if (lane < STRIPES) {
+            st(counter(s, job, 0u, lane), 0u);
+            st(counter(s, job, 1u, lane), 0u);
+        }
+        if (lane == 0) {
+            st(&J.entry, k);
+            st(&J.seed, pair_at(2));
+            st(&J.base, word_at(4));
+        }
+        KIND::install(s, word_at(4));
+    });
     // Claim order: append, or insert before the first larger job (the list
     // is in order of size then).
     const unsigned int listed = lane < n ? ld(&core->active[lane]) : JOBS;
@@ -311,7 +321,6 @@ __device__ HZ_INLINE bool install(const ResidentState& s, unsigned int k, unsign
     unsigned int at = n;
     if (s.policy == SMALLEST_FIRST) at = hz::wave::popc(hz::wave::ballot(lane < n && listed_size <= size));
     if (lane == 0) {
-        st(&J.next, 0u);
         __hip_atomic_fetch_or(&core->open_jobs, 1ull << job, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         st(&core->active[at], job);
         st(&core->active_size[at], size);
@@ -374,7 +383,7 @@ __device__ HZ_INLINE void poll(const ResidentState& s, ResidentClaim& t) {
     unsigned int limit = 0u;
     bool all_claimed = false, finished = false;
     if (job < JOBS) {
-        const unsigned long long both = ld((const unsigned long long*)&core->jobs[job]);
+        const unsigned long long both = ld(&core->jobs[job].claims);
         limit = (unsigned int)(both >> 32);
         all_claimed = (unsigned int)both >= limit;
     }
@@ -434,7 +443,7 @@ __device__ HZ_INLINE void poll(const ResidentState& s, ResidentClaim& t) {
 
 // Gives each lane without items a share of one job's items, from the first
 // job in claim order with items left: the active list, the open set and the
-// jobs' claim counters are read by the lanes in parallel (one round trip when
+// jobs' claim words are read by the lanes in parallel (one round trip when
 // no job is open), then one atomic claims for the whole wavefront, of
 // KIND::per_lane(left, lanes) items per lane (`left` items unclaimed, `lanes`
 // lanes in the launch). Returns false if nothing could be claimed;
@@ -464,7 +473,7 @@ __device__ HZ_INLINE bool claim(const ResidentState& s, ResidentClaim& t, bool& 
     const bool listed = lane < n && slot < JOBS && (open >> slot & 1ull);
     unsigned int seen = 0u, limit = 0u;
     if (listed) {
-        const unsigned long long both = ld((const unsigned long long*)&core->jobs[slot]);
+        const unsigned long long both = ld(&core->jobs[slot].claims);
         seen = (unsigned int)both;
         limit = (unsigned int)(both >> 32);
     }
@@ -482,35 +491,30 @@ __device__ HZ_INLINE bool claim(const ResidentState& s, ResidentClaim& t, bool& 
     while (avail != 0ull) {
         const uint32_t lead = (uint32_t)__builtin_ctzll(avail);
         avail &= avail - 1ull;
-        unsigned int base = 0u, got = 0u, per = 1u;
+        Grant grant{0u, 0u};
+        unsigned int per = 1u;
         if (lane == lead) {
             const unsigned int left = limit - seen;
             per = KIND::per_lane(left > all_left ? left : all_left, gridDim.x * blockDim.x);
             if (KIND::SHARES_OF_ALL && per > 1u && (uint64_t)per * want_lanes > left) {
                 per = (left + want_lanes - 1u) / want_lanes;
             }
-            ResidentJob& J = core->jobs[slot];
-            const unsigned int want = want_lanes * per;
-            const unsigned int old = __hip_atomic_fetch_add(&J.next, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // The job entry may have been replaced since it was read: the
-            // limit that counts is the one read after the claim, below.
-            base = old;
-            got = want;
+            ClaimMemory memory;
+            grant = take_items(memory, &core->jobs[slot].claims, want_lanes * per);
         }
-        const unsigned int job = hz::wave::read_lane(slot, lead);
-        base = hz::wave::read_lane(base, lead);
-        per = hz::wave::read_lane(per, lead);
-        got = hz::wave::read_lane(got, lead);
-        stores_done();
-        // The entry again, in one load, a word per lane: it stays while items
-        // claimed from it are left.
-        const unsigned int word = ld((const unsigned int*)&core->jobs[job] + (lane & 7u));
-        auto word_of = [&](size_t byte) { return hz::wave::read_lane(word, (uint32_t)(byte / 4u)); };
-        const unsigned int lim = word_of(offsetof(ResidentJob, limit));
-        got = base < lim ? (lim - base < got ? lim - base : got) : 0u;
+        const unsigned int got = hz::wave::read_lane(grant.got, lead);
         if (got == 0u) continue;
+        const unsigned int base = hz::wave::read_lane(grant.base, lead);
+        const unsigned int job = hz::wave::read_lane(slot, lead);
+        per = hz::wave::read_lane(per, lead);
         claimed = job;
         bulk = per > 1u;
+        // The entry's fields, after the claim and in one load, a word per
+        // lane: it stays while items claimed from it are left.
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        unsigned int word = 0u;
+        if constexpr (KIND::CLAIMS_SEED) word = ld((const unsigned int*)&core->jobs[job] + (lane & 7u));
+        auto word_of = [&](size_t byte) { return hz::wave::read_lane(word, (uint32_t)(byte / 4u)); };
         if (t.next >= t.end) {
             const unsigned int r = hz::wave::rank(need) * per;
             t.job = job;
