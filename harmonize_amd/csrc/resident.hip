@@ -8,7 +8,7 @@
 // host-coherent ring and advances the ring head. If no launch is running, it
 // launches one; a running launch installs the descriptor at its next
 // housekeeping pass and its groups start claiming the job's items. The launch
-// reports each completion in the ring's completion words, which the host
+// reports each completion in the doorbell's completion words, which the host
 // polls without any HIP call, and ends once it has had no job for idle_us (or
 // once idle after hz_resident_drain); the job table persists, so the next
 // launch carries on.
@@ -178,11 +178,11 @@ struct hz_resident {
     void reap_jobs() {
         for (auto it = in_flight.begin(); it != in_flight.end();) {
             const uint32_t k = it->first;
-            if (__atomic_load_n(&bell->done[k % R::RING], __ATOMIC_ACQUIRE) != k + 1u) {
+            RJob& j = jobs[(size_t)it->second];
+            if (__atomic_load_n(&bell->done[R::completion_word(k, j.table)], __ATOMIC_ACQUIRE) != k + 1u) {
                 ++it;
                 continue;
             }
-            RJob& j = jobs[(size_t)it->second];
             j.status = HZ_JOB_DONE;
             j.end_ms = now_ms(t0);
             table_free |= 1ull << j.table;

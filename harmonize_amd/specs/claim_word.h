@@ -1,5 +1,8 @@
-// The claim word of a job-table entry (specs/resident.h): the items claimed so
-// far in its low half, the items in all in its high half.
+// What groups, housekeeper and host share of a job-table entry
+// (specs/resident.h): its claim word and its completion word.
+//
+// The claim word holds the items claimed so far in its low half and the items
+// in all in its high half.
 //
 // Groups claim from an entry while the housekeeper may be replacing its job,
 // so a claim must not combine one job's counter with another's size. It is one
@@ -55,6 +58,18 @@ HZ_HD inline void replace_job(MEM& mem, unsigned long long* word, unsigned int s
     write_fields();
     mem.wait();
     mem.store(word, claim_word(0u, size));
+}
+
+// The doorbell word in which the kernel reports that ring entry `entry`,
+// installed in job-table entry `job`, has completed. The host gives a table
+// entry to the next job only when it has seen the completion of the last, so
+// the words of jobs in flight are distinct. (Ring positions are not: a large
+// job claimed smallest first is overtaken by more entries than the ring has,
+// and of two jobs in flight a ring's length apart one completion overwrote
+// the other before the host had looked.)
+HZ_HD inline unsigned int completion_word(unsigned int entry, unsigned int job) {
+    (void)entry;
+    return job;
 }
 
 }  // namespace resident

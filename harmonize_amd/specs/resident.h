@@ -8,7 +8,7 @@
 // job table (ResidentCore) and its groups claim work items from the installed
 // jobs in priority order (admission order, or the smallest job first, so a
 // small job overtakes a large one at the next claim). Each job completes on its
-// own and the kernel reports it in the ring's completion words. A kernel with
+// own and the kernel reports it in the doorbell's completion words. A kernel with
 // no job for `idle_ticks` of the device wall clock, or asked by the host to
 // stop once idle, stops claiming and ends; the host relaunches it for later
 // jobs, and the job table carries over between launches.
@@ -87,7 +87,7 @@ struct ResidentDoorbell {
     unsigned int stop;         // 1: stop once idle (host)
     unsigned int consumed;     // entries installed (device)
     unsigned int pad;
-    unsigned int done[hz::resident::RING];      // entry k: k + 1 once its job has completed (device)
+    unsigned int done[hz::resident::JOBS];      // completion_word of entry k: k + 1 once its job has completed (device)
     ResidentEntry entries[hz::resident::RING];  // entry k at k % RING (host)
 };
 
@@ -410,7 +410,7 @@ __device__ HZ_INLINE void poll(const ResidentState& s, ResidentClaim& t) {
             st(&core->completions, ld(&core->completions) + hz::wave::popc(done));
         }
         stores_done();
-        if (finished) sys_st(&s.bell->done[entry % RING], entry + 1u);
+        if (finished) sys_st(&s.bell->done[completion_word(entry, job)], entry + 1u);
         hz::wave::sync();
     }
 

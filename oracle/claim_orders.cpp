@@ -1,5 +1,8 @@
 // ORACLE — test infrastructure only (see host_shim.h).
 //
+// What groups, housekeeper and host share of the resident program's job table
+// (specs/claim_word.h), on the host.
+//
 // Every order of the memory accesses of two groups that claim from a
 // job-table entry of the resident program while the housekeeper replaces the
 // entry's job. The accesses are those of specs/claim_word.h, or of the
@@ -165,6 +168,38 @@ bool order_is_right(bool planted, std::vector<std::pair<int, int>>& choices) {
 }
 
 }  // namespace
+
+// Jobs all there at once, served by a table of `table` entries that the host
+// fills in order, smallest installed job first: how many pairs of jobs that
+// are in flight together report in the same completion word. `ring` is 0 for
+// the runtime's words, or the length of a ring whose positions are the words
+// (the planted mistake).
+extern "C" uint64_t oracle_shared_completion_words(const uint32_t* sizes, uint32_t jobs, uint32_t table,
+                                                   uint32_t ring) {
+    struct Flight {
+        uint32_t entry, job;
+    };
+    std::vector<Flight> flying;
+    std::vector<uint32_t> free_entries;
+    for (uint32_t t = table; t > 0; --t) free_entries.push_back(t - 1u);
+    auto word = [&](const Flight& f) { return ring ? f.entry % ring : hz::resident::completion_word(f.entry, f.job); };
+    uint64_t shared = 0;
+    for (uint32_t next = 0; next < jobs || !flying.empty();) {
+        while (next < jobs && !free_entries.empty()) {
+            const Flight f{next++, free_entries.back()};
+            free_entries.pop_back();
+            for (const Flight& o : flying) shared += word(o) == word(f);
+            flying.push_back(f);
+        }
+        size_t least = 0;
+        for (size_t i = 1; i < flying.size(); ++i) {
+            if (sizes[flying[i].entry] < sizes[flying[least].entry]) least = i;
+        }
+        free_entries.push_back(flying[least].job);
+        flying.erase(flying.begin() + (long)least);
+    }
+    return shared;
+}
 
 // Runs every order; returns how many there are, and in *wrong how many of
 // them grant an item twice, not at all, or with another job's fields.
