@@ -12,9 +12,10 @@ bounded sample of the same workload). Further sections: the photon walk and
 the batched BFS (Async vs Event), the futures tree, the remapping-barrier demo
 and the serving load sweep (p50/p99 latency at 20-100% of peak).
 
-Consistency checks made here (a failure raises): the Collatz step counts of
-AsyncProgram, EventProgram and the one-thread-per-start kernel are identical;
-photon event totals and BFS levels agree between the two programs; the futures
+Consistency checks made here: the Collatz step counts of AsyncProgram,
+EventProgram and the one-thread-per-start kernel are identical (a failure
+raises: no line is printed). A further section that fails is named in the line
+("failed"), the sections after it are not run, and the exit status is 1: photon event totals and BFS levels agree between the two programs; the futures
 total and the barrier demo's count match their closed forms. The GPU tests
 check every workload, serving included, against the oracle.
 
@@ -31,6 +32,7 @@ import os
 import platform
 import sys
 import time
+import traceback
 from pathlib import Path
 
 import numpy as np
@@ -509,6 +511,20 @@ LEGS = {
 }
 
 
+def run_sections(out: dict, sections: list) -> None:
+    """Runs (name, function) pairs into out[name]. The first that raises is
+    recorded in out["failed"], and those after it are not run (it may have left
+    the device unusable) but listed there."""
+    for k, (name, run) in enumerate(sections):
+        try:
+            out[name] = run()
+        except Exception as e:
+            traceback.print_exc()
+            out["failed"] = {"section": name, "error": str(e), "not_run": [n for n, _ in sections[k + 1:]]}
+            return
+        progress(name)
+
+
 def main() -> int:
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("--gpus", type=int, default=1)
@@ -649,26 +665,6 @@ def main() -> int:
         out["async_vs_event"] = value / out["event"]["value"]
         progress("Collatz EventProgram")
 
-    if not args.no_photon:
-        out["photon"] = photon_comparison(hz)
-        progress("photon walk")
-
-    if not args.no_bfs:
-        out["bfs"] = bfs_comparison(hz)
-        progress("BFS batch")
-
-    if not args.no_futures:
-        out["futures"] = futures_comparison(hz)
-        progress("futures tree")
-    if not args.no_barrier:
-        out["barrier"] = barrier_demo(hz)
-        progress("barrier demo")
-
-    if not args.no_serve:
-        out["serving"] = serving_sweep(hz)
-        out["serving_resident"] = resident_sweep(hz)
-        out["serving_resident_photon"] = resident_sweep(hz, "photon")
-
     pl = hz.collatz_run("plain", steps_out, starts, COUNT)
     if not np.array_equal(steps_out.numpy(), steps_async):
         raise RuntimeError("collatz: AsyncProgram and one-thread-per-start step counts differ")
@@ -678,12 +674,19 @@ def main() -> int:
         "note": "one thread per start, no runtime (steps computed per second, same work)",
     }
 
-    if not args.no_cpu:
-        out["cpu_baseline"] = cpu_baseline()
-        progress("CPU baseline")
-
+    sections = [
+        ("photon", not args.no_photon, lambda: photon_comparison(hz)),
+        ("bfs", not args.no_bfs, lambda: bfs_comparison(hz)),
+        ("futures", not args.no_futures, lambda: futures_comparison(hz)),
+        ("barrier", not args.no_barrier, lambda: barrier_demo(hz)),
+        ("serving", not args.no_serve, lambda: serving_sweep(hz)),
+        ("serving_resident", not args.no_serve, lambda: resident_sweep(hz)),
+        ("serving_resident_photon", not args.no_serve, lambda: resident_sweep(hz, "photon")),
+        ("cpu_baseline", not args.no_cpu, cpu_baseline),
+    ]
+    run_sections(out, [(name, run) for name, wanted, run in sections if wanted])
     print(json.dumps(out), flush=True)
-    return 0
+    return 1 if "failed" in out else 0
 
 
 if __name__ == "__main__":
