@@ -93,7 +93,8 @@ struct AtomicIter {
     __device__ bool sync_done() const { return done(); }
 };
 
-// A lane's share of a claimed range: next, next + stride, ... below end.
+// A lane's share of a claimed range: next, next + stride, ... below end. No
+// index beyond end is formed, so that end may be the type's greatest value.
 template <typename INDEX_TYPE>
 struct Share {
     INDEX_TYPE next;
@@ -109,8 +110,15 @@ struct Share {
     HZ_HD bool step(INDEX_TYPE& index) {
         if (next >= end) return false;
         index = next;
-        next += stride;
+        next = end - next > stride ? next + stride : end;
         return true;
+    }
+
+    // The share of lane r of n in [first, limit).
+    HZ_HD void take(INDEX_TYPE first, INDEX_TYPE limit, INDEX_TYPE r, INDEX_TYPE n) {
+        next = first < limit && r < limit - first ? first + r : limit;
+        end = limit;
+        stride = n;
     }
 };
 
@@ -144,19 +152,20 @@ __device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TY
     const uint64_t all = (uint64_t)gridDim.x * blockDim.x;
     uint64_t per = (uint64_t)(limit - at) / all;
     per = per > most ? most : per;
-    // (Near the top of the type, small claims keep the counter from wrapping.)
-    if (per < 1 || limit - at < from || limit > (INDEX_TYPE)0xF0000000u) per = 1;
+    if (per < 1 || limit - at < from) per = 1;
     const INDEX_TYPE total = n * (INDEX_TYPE)per;
+    // Claims that add their whole size move the counter past the end, each
+    // resident wavefront by at most 64 shares of `most` (17 million for 32 and
+    // 8,192 wavefronts). Where that could wrap it, claims stop at the end.
     INDEX_TYPE base = 0;
-    if (need && r == 0) base = hz::wave::atomic_add(&range.value, total);
+    if (need && r == 0) {
+        base = limit > (INDEX_TYPE)0xF0000000u ? hz::wave::claim_below(&range.value, total, limit)
+                                               : hz::wave::atomic_add(&range.value, total);
+    }
     base = (INDEX_TYPE)hz::wave::read_lane((uint32_t)base, (uint32_t)__builtin_ctzll(lanes));
     INDEX_TYPE end = base + total;
     if (end < base || end > limit) end = limit;
-    if (need) {
-        share.next = base < limit ? base + r : limit;
-        share.end = end;
-        share.stride = n;
-    }
+    if (need) share.take(base, end, r, n);
 #else
     (void)most;
     (void)from;

@@ -124,6 +124,21 @@ __device__ HZ_INLINE T aggregated_fetch_add(T* counter, T amount) {
     return atomic_add(counter, amount);
 }
 
+// Claims up to `want` below `limit` by one lane: returns the counter before,
+// and never moves it past the limit.
+template <typename T>
+__device__ HZ_INLINE T claim_below(T* counter, T want, T limit) {
+    T at = atomic_load(counter);
+    while (at < limit) {
+        const T next = limit - at > want ? at + want : limit;
+        if (__hip_atomic_compare_exchange_strong(counter, &at, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT)) {
+            break;
+        }
+    }
+    return at;
+}
+
 }  // namespace wave
 }  // namespace hz
 

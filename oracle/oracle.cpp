@@ -125,6 +125,26 @@ void oracle_collatz_make_starts(uint64_t seed, uint32_t bits, uint32_t count, ui
     }
 }
 
+// Marks what each of n lanes steps through of its share of [first, limit)
+// (util::iter::Share): marks[i - first] counts visits of index i. Returns the
+// indices visited outside the range.
+uint64_t oracle_share_steps(uint32_t first, uint32_t limit, uint32_t n, uint32_t* marks) {
+    uint64_t outside = 0;
+    for (uint32_t r = 0; r < n; ++r) {
+        util::iter::Share<unsigned int> share;
+        share.take(first, limit, r, n);
+        unsigned int index;
+        for (uint64_t k = 0; share.step(index) && k <= 1u << 16; ++k) {
+            if (index < first || index >= limit) {
+                outside++;
+            } else {
+                marks[index - first]++;
+            }
+        }
+    }
+    return outside;
+}
+
 int oracle_max_threads(void) { return omp_get_max_threads(); }
 
 // Photon-walk parameters, laid out as hz_photon_params in harmonize_amd.h.
