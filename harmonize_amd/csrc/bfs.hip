@@ -40,7 +40,7 @@ namespace {
 struct DeviceBytes {
     void* p = nullptr;
     DeviceBytes() = default;
-    explicit DeviceBytes(size_t bytes) { check(hipMalloc(&p, bytes ? bytes : 1), "hipMalloc(bfs)"); }
+    explicit DeviceBytes(size_t bytes) { check(util::host::device_malloc(&p, bytes ? bytes : 1), "hipMalloc(bfs)"); }
     ~DeviceBytes() {
         if (p) (void)hipFree(p);
     }
@@ -97,18 +97,14 @@ struct hz_bfs_batch {
     hipStream_t stream = nullptr;
     double build_ms = 0.0;
     std::map<std::vector<uint64_t>, std::unique_ptr<Runner>> runners;
-    // EventProgram's instance, kept like the async runners: its queues hold
-    // gigabytes for a large batch, which cost 1.5 ms or, after an idle spell,
-    // a hundred to allocate and free on every search.
-    std::unique_ptr<BfsEventHints::Instance> event_instance;
-    uint64_t event_io = 0;
-    std::unique_ptr<hz::capi::HostCell<BfsEventHints::Header>> event_header;
 
     ~hz_bfs_batch() {
         runners.clear();
-        event_instance.reset();
+        release_event_space();
         if (stream) (void)hipStreamDestroy(stream);
     }
+
+    void release_event_space();
 
     void layout(const uint32_t* v, const uint64_t* e, const uint32_t* src) {
         vertices.assign(v, v + graphs);
@@ -273,6 +269,42 @@ struct AsyncRunner : Runner {
     }
 };
 
+// EventProgram's instance and header, kept by the batch between its searches:
+// the queues hold gigabytes for a large batch, which cost 1.5 ms or, after an
+// idle spell, a hundred to allocate and free on every search. A batch keeps up
+// to KEPT_BYTES; idle, they are freed like other workspaces when an allocation
+// fails.
+using BfsEventSpace = hz::capi::EventSpace<BfsEventHints>;
+constexpr uint64_t KEPT_BYTES = 8ull << 30;
+const char EVENT_SPACE = 0;  // its address names the kind
+
+struct EventSpaceHold {
+    hz_bfs_batch& b;
+    const uint64_t io;
+    const int exceptions = std::uncaught_exceptions();
+    std::unique_ptr<BfsEventSpace> space;
+
+    EventSpaceHold(hz_bfs_batch& batch, uint64_t size) : b(batch), io(size) {
+        space.reset(static_cast<BfsEventSpace*>(hz::capi::workspace_take(&EVENT_SPACE, io, (uint64_t)&b).release()));
+        if (space) return;
+        b.release_event_space();  // one of another size
+        try {
+            space = std::make_unique<BfsEventSpace>(io, 0);
+        } catch (const std::exception&) {
+            // Allocations have freed the idle workspaces; the batch's async
+            // runners are left.
+            if (b.runners.empty()) throw;
+            (void)hipGetLastError();
+            b.runners.clear();
+            space = std::make_unique<BfsEventSpace>(io, 0);
+        }
+    }
+    ~EventSpaceHold() {
+        if (std::uncaught_exceptions() > exceptions || space->bytes() > KEPT_BYTES) return;
+        hz::capi::workspace_keep(&EVENT_SPACE, io, (uint64_t)&b, std::move(space));
+    }
+};
+
 void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     uint64_t io = c.arena;
     if (io == 0) {
@@ -281,12 +313,8 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
         if (io < (1ull << 20)) io = 1ull << 20;
         if (io > (1ull << 30)) io = 1ull << 30;
     }
-    if (!b.event_instance || b.event_io != io) {
-        b.event_instance.reset();
-        b.event_instance = std::make_unique<BfsEventHints::Instance>(io, b.state(default_split(c)));
-        b.event_io = io;
-    }
-    BfsEventHints::Instance& inst = *b.event_instance;
+    EventSpaceHold hold(b, io);
+    BfsEventHints::Instance& inst = hold.space->inst;
     inst.device_state = b.state(default_split(c));
     inst.reset(b.stream);
     // 16 groups per CU: measured 22.2 ms on the 64-graph batch against 23.7
@@ -297,9 +325,8 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     StreamTimer t(b.stream);
     t.start();
     b.enqueue_reset();
-    if (!b.event_header) b.event_header = std::make_unique<hz::capi::HostCell<BfsEventHints::Header>>();
     const uint64_t launches =
-        hz::capi::run_generations<BfsEventHints>(inst, groups, chunk, max_launches, b.stream, b.event_header->p);
+        hz::capi::run_generations<BfsEventHints>(inst, groups, chunk, max_launches, b.stream, hold.space->header.p);
     double ms = t.stop();
     if (stats) {
         auto s = inst.read_status();
@@ -343,6 +370,12 @@ std::unique_ptr<Runner> make_async_runner(hz_bfs_batch& b, const hz_run_config& 
             throw std::invalid_argument("hz_bfs_batch_run: stash must be 8 or 16 links");
     }
 }
+
+}  // namespace
+
+void hz_bfs_batch::release_event_space() { hz::capi::workspace_drop(&EVENT_SPACE, (uint64_t)this); }
+
+namespace {
 
 void check_batch(const hz_bfs_batch* b) {
     if (!b) throw std::invalid_argument("hz_bfs: null batch");
@@ -511,8 +544,7 @@ extern "C" int hz_bfs_batch_run(hz_bfs_batch* batch, int kind, const hz_run_conf
                 } catch (const std::exception&) {
                     // Room taken by what earlier runs left behind.
                     (void)hipGetLastError();
-                    if (hz::capi::workspace_release() == 0 && !batch->event_instance) throw;
-                    batch->event_instance.reset();
+                    if (hz::capi::workspace_release() == 0) throw;
                     made = make_async_runner(*batch, c);
                 }
                 it = batch->runners.emplace(key, std::move(made)).first;
@@ -528,6 +560,6 @@ extern "C" int hz_bfs_batch_release(hz_bfs_batch* batch) {
     return guarded([&] {
         check_batch(batch);
         batch->runners.clear();
-        batch->event_instance.reset();
+        batch->release_event_space();
     });
 }

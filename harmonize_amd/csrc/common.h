@@ -83,7 +83,7 @@ struct DeviceIter {
     util::iter::AtomicIter<unsigned int>* ptr = nullptr;
     explicit DeviceIter(unsigned int limit) {
         util::iter::AtomicIter<unsigned int> host(0u, limit);
-        check(hipMalloc((void**)&ptr, sizeof(host)), "hipMalloc(iterator)");
+        check(util::host::device_malloc((void**)&ptr, sizeof(host)), "hipMalloc(iterator)");
         check(hipMemcpy(ptr, &host, sizeof(host), hipMemcpyHostToDevice), "hipMemcpy(iterator)");
     }
     ~DeviceIter() {
@@ -177,7 +177,7 @@ uint64_t run_generations(typename P::Instance& inst, uint32_t groups, uint32_t c
     }                                                                                                   \
     extern "C" void* alloc_state_##suffix(void) {                                                       \
         void* p = nullptr;                                                                              \
-        hz::capi::guarded([&] { hz::capi::check(hipMalloc(&p, sizeof(STATE)), "hipMalloc(state)"); });   \
+        hz::capi::guarded([&] { hz::capi::check(util::host::device_malloc(&p, sizeof(STATE)), "hipMalloc(state)"); }); \
         return p;                                                                                       \
     }                                                                                                   \
     extern "C" void free_state_##suffix(void* state) {                                                  \

@@ -39,20 +39,18 @@ extern "C" const char* hz_last_error(void) {
 
 extern "C" void* harmonize_alloc_device_bytes(size_t size) {
     void* p = nullptr;
-    guarded([&] {
-        hipError_t e = hipMalloc(&p, size);
-        if (e != hipSuccess && hz::capi::workspace_release() != 0) {
-            (void)hipGetLastError();
-            e = hipMalloc(&p, size);
-        }
-        check(e, "hipMalloc");
-    });
+    guarded([&] { check(util::host::device_malloc(&p, size), "hipMalloc"); });
     return p;
 }
 
 extern "C" void* harmonize_alloc_managed_bytes(size_t size) {
     void* p = nullptr;
-    guarded([&] { check(hipMallocManaged(&p, size), "hipMallocManaged"); });
+    guarded([&] {
+        hipError_t e = hipMallocManaged(&p, size);
+        if (e != hipSuccess) (void)hipGetLastError();
+        if (e == hipErrorOutOfMemory && hz::capi::workspace_release() != 0) e = hipMallocManaged(&p, size);
+        check(e, "hipMallocManaged");
+    });
     return p;
 }
 

@@ -346,8 +346,9 @@ extern "C" int hz_resident_create(const hz_resident_config* config, hz_resident*
               "hipHostMalloc(doorbell)");
         std::memset(r->bell, 0, sizeof(ResidentDoorbell));
         check(hipHostGetDevicePointer((void**)&r->bell_dev, r->bell, 0), "hipHostGetDevicePointer");
-        check(hipMalloc((void**)&r->core, sizeof(ResidentCore)), "hipMalloc(resident core)");
-        check(hipMalloc((void**)&r->counters, sizeof(unsigned int) * R::COUNTER_WORDS), "hipMalloc(counters)");
+        check(util::host::device_malloc((void**)&r->core, sizeof(ResidentCore)), "hipMalloc(resident core)");
+        check(util::host::device_malloc((void**)&r->counters, sizeof(unsigned int) * R::COUNTER_WORDS),
+              "hipMalloc(counters)");
         // The item space, indexed by u32: 12 bytes per Collatz item (a u64
         // start and a u32 count); for photon jobs 4 bytes per photon (its
         // event count) plus the job's tally, 8 x tally_stride bytes.
@@ -355,8 +356,10 @@ extern "C" int hz_resident_create(const hz_resident_config* config, hz_resident*
         r->capacity = c.pool_bytes / (photon ? 4ull : 12ull);
         if (r->capacity > 0xFFFFFF00ull) r->capacity = 0xFFFFFF00ull;
         if (r->capacity < 256) throw std::invalid_argument("hz_resident_create: pool_bytes too small");
-        if (!photon) check(hipMalloc((void**)&r->starts, 8ull * r->capacity), "hipMalloc(resident starts)");
-        check(hipMalloc((void**)&r->steps, 4ull * r->capacity), "hipMalloc(resident outputs)");
+        if (!photon) {
+            check(util::host::device_malloc((void**)&r->starts, 8ull * r->capacity), "hipMalloc(resident starts)");
+        }
+        check(util::host::device_malloc((void**)&r->steps, 4ull * r->capacity), "hipMalloc(resident outputs)");
         r->pool = std::make_unique<Pool>(r->capacity);
         hz_photon_params pp{};
         hz_photon_defaults(&pp);

@@ -541,7 +541,7 @@ extern "C" int hz_server_create(const hz_server_config* config, hz_server** out)
         if (c.slots > 8) throw std::invalid_argument("hz_server_create: at most 8 slots");
         if (c.arena_links == 0) c.arena_links = 1ull << 16;
         s->t0 = std::chrono::steady_clock::now();
-        check(hipMalloc(&s->pool_base, c.pool_bytes), "hipMalloc(serve pool)");
+        check(util::host::device_malloc(&s->pool_base, c.pool_bytes), "hipMalloc(serve pool)");
         s->pool = std::make_unique<Pool>(c.pool_bytes);
         s->groups_collatz = share_of<SCollatz>(c.slots);
         s->groups_photon = share_of<SPhoton>(c.slots);

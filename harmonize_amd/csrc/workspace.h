@@ -8,8 +8,11 @@
 // sizes on its device. A call owns its workspace alone while it runs, so
 // calls of several threads each have one; it is cleared by kernels before
 // use. Idle workspaces hold at most IDLE_BYTES over all devices, the ones
-// idle longest are freed first, all of them when an allocation fails or on
-// hz_workspace_release(); a call that failed frees its own.
+// idle longest are freed first, all of them when a device allocation of this
+// library fails (util::host::device_malloc) or on hz_workspace_release(); a
+// call that failed frees its own. An object that keeps a workspace for its own
+// calls (a BFS batch) leaves it on the same shelf, so that it too is freed
+// when memory runs short, but beside the bound.
 #pragma once
 
 #include <exception>
@@ -30,6 +33,10 @@ struct Workspace {
 std::unique_ptr<Workspace> workspace_take(const void* kind, uint64_t a, uint64_t b);
 // Keeps a workspace for later calls (or frees it, or others, at the bound).
 void workspace_give(const void* kind, uint64_t a, uint64_t b, uint64_t bytes, std::unique_ptr<Workspace> w) noexcept;
+// Keeps a workspace for the object that `b` names, beside the bound.
+void workspace_keep(const void* kind, uint64_t a, uint64_t b, std::unique_ptr<Workspace> w) noexcept;
+// Frees the idle workspaces of a kind that are kept for the object `b`.
+void workspace_drop(const void* kind, uint64_t b) noexcept;
 // Frees every idle workspace; returns how many there were.
 size_t workspace_release();
 
@@ -44,6 +51,7 @@ class Lease {
         try {
             w_ = std::make_unique<W>(a, b);
         } catch (const std::exception&) {
+            // Host memory, events: freeing idle workspaces may help there too.
             (void)hipGetLastError();
             if (workspace_release() == 0) throw;
             w_ = std::make_unique<W>(a, b);
@@ -70,7 +78,7 @@ class Lease {
 struct Scratch : Workspace {
     unsigned char* p = nullptr;
     uint64_t size;
-    Scratch(uint64_t bytes, uint64_t) : size(bytes ? bytes : 1) { check(hipMalloc((void**)&p, size), "hipMalloc(scratch)"); }
+    Scratch(uint64_t bytes, uint64_t) : size(bytes ? bytes : 1) { check(util::host::device_malloc((void**)&p, size), "hipMalloc(scratch)"); }
     ~Scratch() override {
         if (p) (void)hipFree(p);
     }

@@ -13,7 +13,7 @@ struct Idle {
     const void* kind;
     uint64_t a, b;
     int device;
-    uint64_t bytes;
+    uint64_t bytes;  // counted against the bound (0: kept for an object)
     std::unique_ptr<Workspace> w;
 };
 
@@ -65,9 +65,32 @@ void workspace_give(const void* kind, uint64_t a, uint64_t b, uint64_t bytes, st
         return;
     }
     s.bytes += bytes;
-    while (s.bytes > IDLE_BYTES) {
-        s.bytes -= s.idle.back().bytes;
-        old.splice(old.begin(), s.idle, std::prev(s.idle.end()));
+    for (auto it = s.idle.end(); s.bytes > IDLE_BYTES && it != s.idle.begin();) {
+        auto last = std::prev(it);
+        if (last->bytes == 0) {
+            it = last;
+            continue;
+        }
+        s.bytes -= last->bytes;
+        old.splice(old.begin(), s.idle, last);
+    }
+}
+
+void workspace_keep(const void* kind, uint64_t a, uint64_t b, std::unique_ptr<Workspace> w) noexcept {
+    workspace_give(kind, a, b, 0, std::move(w));
+}
+
+void workspace_drop(const void* kind, uint64_t b) noexcept {
+    std::list<Idle> old;  // freed after the lock
+    Shelf& s = shelf();
+    std::lock_guard<std::mutex> lock(s.mutex);
+    for (auto it = s.idle.begin(); it != s.idle.end();) {
+        auto next = std::next(it);
+        if (it->kind == kind && it->b == b) {
+            s.bytes -= it->bytes;
+            old.splice(old.begin(), s.idle, it);
+        }
+        it = next;
     }
 }
 
@@ -83,6 +106,12 @@ size_t workspace_release() {
 }
 
 namespace {
+// Device allocations that fail free the idle workspaces and try again.
+const bool hooked = [] {
+    util::host::free_idle_memory = [] { return workspace_release() != 0; };
+    return true;
+}();
+
 __global__ void __launch_bounds__(64) set_iter_kernel(util::iter::AtomicIter<unsigned int>* it, unsigned int limit) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *it = util::iter::AtomicIter<unsigned int>(0u, limit);
 }

@@ -79,11 +79,28 @@ inline void auto_throw(hipError_t status) {
     }
 }
 
+// Frees device memory that is kept for later use, and says whether there was
+// any; set by the runtime library, which keeps the workspaces of its runs.
+inline bool (*free_idle_memory)() = nullptr;
+
+// hipMalloc, tried again once idle memory has been freed. A failure is
+// returned only: left as the thread's last error, also by an attempt before one
+// that succeeds, it would be taken for that of a later launch.
+inline hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e == hipErrorOutOfMemory && free_idle_memory != nullptr && free_idle_memory()) {
+        e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+    }
+    return e;
+}
+
 template <typename T>
 T* hardMalloc(size_t size) {
     T* result = nullptr;
     if (size == 0) return nullptr;
-    auto_throw(hipMalloc((void**)&result, sizeof(T) * size));
+    auto_throw(device_malloc((void**)&result, sizeof(T) * size));
     return result;
 }
 

@@ -498,7 +498,9 @@ int hz_bfs_batch_layout(const hz_bfs_batch* batch, uint32_t* vertices, uint64_t*
 /* BFS of every job of the batch in one program (kind HZ_ASYNC or HZ_EVENT);
  * levels land in info.d_level. */
 int hz_bfs_batch_run(hz_bfs_batch* batch, int kind, const hz_run_config* config, hz_run_stats* stats);
-/* Frees the program instances the batch keeps for reuse. */
+/* Frees the program instances the batch keeps for reuse: one for each HZ_ASYNC
+ * configuration it has run, and that of HZ_EVENT up to 8 GiB, which is also
+ * freed when a device allocation fails. */
 int hz_bfs_batch_release(hz_bfs_batch* batch);
 
 /* ------------------------------------------------------------ autotuning
@@ -747,8 +749,9 @@ int hz_device_synchronize(void);
 
 /* A hz_*_run call that ends well leaves its device workspace (program
  * instance, arena, queues) for the next call of its kind and sizes on that
- * device; idle workspaces hold at most 1 GiB in all. This frees them now. An
- * allocation that fails frees them by itself. */
+ * device; idle workspaces hold at most 1 GiB in all. This frees them now, and
+ * those that BFS batches keep. A device allocation of this library that fails
+ * frees them by itself and is tried again. */
 int hz_workspace_release(void);
 
 /* Device-to-device copy of `bytes` bytes, synchronous (used to calibrate
