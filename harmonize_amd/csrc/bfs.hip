@@ -326,7 +326,8 @@ void run_event(hz_bfs_batch& b, const hz_run_config& c, hz_run_stats* stats) {
     t.start();
     b.enqueue_reset();
     const uint64_t launches =
-        hz::capi::run_generations<BfsEventHints>(inst, groups, chunk, max_launches, b.stream, hold.space->header.p);
+        hz::capi::run_generations<BfsEventHints>(inst, groups, c.groups == 0, chunk, max_launches, b.stream,
+                                                 hold.space->header.p);
     double ms = t.stop();
     if (stats) {
         auto s = inst.read_status();

@@ -39,7 +39,7 @@ void run_event_chase(ChaseState st, uint32_t lists, const hz_run_config& cfg, hz
     }
     hz::capi::Lease<hz::capi::EventSpace<P>> ws(io, 0);
     st.list_iter = ws->parts.set_iter(lists);
-    ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
+    ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg, stats);
 }
 
 }  // namespace

@@ -102,7 +102,7 @@ extern "C" int hz_collatz_run(int kind, const uint64_t* d_starts, uint32_t count
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
             hz::capi::Lease<hz::capi::EventSpace<CollatzEvent>> ws(io, 0);
             ds.iterator = ws->parts.set_iter(count);
-            ws->run(ds, groups, chunk, cfg.max_launches, stats);
+            ws->run(ds, groups, chunk, cfg, stats);
         } else {
             throw std::invalid_argument("hz_collatz_run: unknown program kind");
         }

@@ -101,7 +101,7 @@ extern "C" int hz_futures_run(int kind, const uint64_t* d_starts, uint32_t leave
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
             hz::capi::Lease<hz::capi::EventSpace<FuturesEvent>> ws(io, 0);
             st.iter = ws->parts.set_iter(leaves + readers);
-            ws->run(st, groups, chunk, cfg.max_launches, stats);
+            ws->run(st, groups, chunk, cfg, stats);
         }
 
         TotalFuture host_total;

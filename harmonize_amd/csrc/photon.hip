@@ -91,7 +91,7 @@ extern "C" int hz_photon_run(int kind, const hz_photon_params* params, double* d
             uint32_t chunk = cfg.cycles ? cfg.cycles : 4u;
             hz::capi::Lease<hz::capi::EventSpace<PhotonEvent>> ws(io, 0);
             st.iterator = ws->parts.set_iter(p.photons);
-            ws->run(st, groups, chunk, cfg.max_launches, stats);
+            ws->run(st, groups, chunk, cfg, stats);
         } else {
             throw std::invalid_argument("hz_photon_run: kind must be HZ_EVENT or HZ_ASYNC");
         }

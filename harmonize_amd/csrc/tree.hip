@@ -56,7 +56,7 @@ extern "C" int hz_tree_run(int kind, int order, uint32_t roots, uint32_t fanout,
             uint64_t io = cfg.arena ? cfg.arena : (1ull << 24);
             hz::capi::Lease<hz::capi::EventSpace<TreeEvent>> ws(io, 0);
             st.root_iter = ws->parts.set_iter(roots);
-            ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg.max_launches, stats);
+            ws->run(st, groups, cfg.cycles ? cfg.cycles : 4u, cfg, stats);
         } else if (kind == HZ_ASYNC) {
             switch (order) {
                 case HZ_TREE_FLAT: run_tree_async<TreeFlatAsync>(st, roots, cfg, stats); break;

@@ -197,14 +197,16 @@ struct EventSpace : Workspace {
     EventSpace(uint64_t io, uint64_t) : inst(io, typename P::DeviceState{}) {}
     uint64_t bytes() const { return 4ull * (inst.queue_a.size() + inst.queue_b.size()); }
 
-    // Runs the program of `state`, its iterator set, generation by generation.
-    void run(const typename P::DeviceState& state, uint32_t groups, uint32_t chunk, uint32_t max_launches,
+    // Runs the program of `state`, its iterator set, generation by generation,
+    // on the caller's number of groups or on up to `groups` of them.
+    void run(const typename P::DeviceState& state, uint32_t groups, uint32_t chunk, const hz_run_config& cfg,
              hz_run_stats* stats) {
         inst.device_state = state;
         inst.reset(nullptr);
         parts.timer.start();
         const uint64_t launches =
-            run_generations<P>(inst, groups, chunk, max_launches ? max_launches : 1u << 24, nullptr, header.p);
+            run_generations<P>(inst, groups, cfg.groups == 0, chunk, cfg.max_launches ? cfg.max_launches : 1u << 24,
+                               nullptr, header.p);
         parts.timer.mark();
         if (stats) {
             auto s = inst.read_status();

@@ -121,6 +121,7 @@ class EventProgram {
         unsigned int* queues[2];  // each [OPS][WORDS][capacity]
         unsigned int capacity;    // per operation, SEGMENTS * seg_capacity
         unsigned int seg_capacity;
+        unsigned int most_links;  // a launch leaves a generation of more input links to a later one (0: never)
     };
 
     // Owns the queues and status of one program instance (reference
@@ -134,6 +135,11 @@ class EventProgram {
         util::host::DevBuf<unsigned int> queue_b;
         DeviceState device_state;
         Status host_status{};
+        // For hosts that launch generations ahead, with groups for what they
+        // last saw: a launch that finds more input links than this does
+        // nothing, so that a generation that has grown waits for a launch of
+        // its size. 0: every launch runs its generation.
+        unsigned int most_links = 0;
 
         static unsigned int seg_cap_for(size_t io_size) {
             if (io_size == 0 || io_size > 0x7FFFFFFFu) {
@@ -159,6 +165,7 @@ class EventProgram {
             result.queues[1] = queue_b.data();
             result.capacity = capacity;
             result.seg_capacity = seg_capacity;
+            result.most_links = most_links;
             return result;
         }
 
@@ -226,6 +233,12 @@ class EventProgram {
     }
 
     __device__ Segment& segment(OpDisc op, uint32_t s) { return _dev_ctx.status->seg[op][s]; }
+
+    // Whether the generation, of `links` input links, is too large for this
+    // launch (DeviceContext::most_links).
+    __device__ static bool left_to_later(const DeviceContext& ctx, unsigned long long links) {
+        return ctx.most_links != 0u && links > ctx.most_links;
+    }
 
     __device__ uint32_t home_segment() const { return blockIdx.x % SEGMENTS; }
 
@@ -339,6 +352,9 @@ class EventProgram {
         _thd_ctx.rand_state = _thd_ctx.thread_id;
         Status* st = _dev_ctx.status;
         const unsigned int in = st->toggle;
+        unsigned long long all = 0;
+        for (uint32_t op = 0; op < OPS; ++op) all += st->links[op];
+        if (left_to_later(_dev_ctx, all)) return;
         _grp_ctx.toggle = in;
         hz::wave::sync();
         const uint32_t home = home_segment();
@@ -417,12 +433,25 @@ class EventProgram {
     __device__ static void flip(DeviceContext ctx) {
         Status* st = ctx.status;
         const uint32_t lane = hz::wave::lane();
-        unsigned long long executed = 0;
+        unsigned long long executed = 0, all = 0;
         uint32_t produced = 0;
+        // The counts are read together: a generation of few promises is one
+        // trip to memory after another.
+        constexpr uint32_t AHEAD = OPS1 < 8u ? OPS1 : 8u;
+        uint32_t came[AHEAD], went[AHEAD];
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; ++i) {
+            came[i] = st->in_count[i][lane];
+            went[i] = st->seg[i][lane].out_count;
+        }
+        for (uint32_t i = 0; i < OPS; ++i) all += st->links[i];
+        if (left_to_later(ctx, all)) return;
+#pragma unroll 8
         for (uint32_t i = 0; i < OPS; ++i) {
             Segment& g = st->seg[i][lane];
-            executed += st->in_count[i][lane];
-            const uint32_t n = g.out_count < ctx.seg_capacity ? g.out_count : ctx.seg_capacity;
+            executed += i < AHEAD ? came[i < AHEAD ? i : 0u] : st->in_count[i][lane];
+            const uint32_t out = i < AHEAD ? went[i < AHEAD ? i : 0u] : g.out_count;
+            const uint32_t n = out < ctx.seg_capacity ? out : ctx.seg_capacity;
             g.out_count = 0;
             g.halt = 0;
             // Links before this lane's segment: an inclusive scan, less its own.
