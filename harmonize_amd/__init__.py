@@ -106,6 +106,8 @@ _SIGNATURES = {
     ),
     "hz_collatz_make_starts": (ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, _VP]),
     "hz_audit_selftest": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_size_t]),
+    "hz_wait_selftest": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32,
+                                        ctypes.POINTER(ctypes.c_uint32)]),
     "hz_tune_cache_set_path": (ctypes.c_int, [ctypes.c_char_p]),
     "hz_tune_cache_lookup": (ctypes.c_int, [ctypes.c_char_p, ctypes.POINTER(RunConfig),
                                             ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)]),

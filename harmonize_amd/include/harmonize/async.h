@@ -426,7 +426,10 @@ class AsyncProgram {
     static_assert(CHAIN_PASSES >= 1 && CHAIN_PASSES <= 16, "CHAIN_PASSES must be in [1, 16]");
     // Evaluations without a refill after which lanes that go on chaining
     // make room for what waits in the stash, so that promises that requeue
-    // themselves until another promise has run cannot keep it waiting.
+    // themselves until another promise has run cannot keep it waiting. A
+    // group whose lanes are nearly all held, and whose stash holds no full
+    // link, then looks at its home queue and for new work too (as it would
+    // between links of less than 64 promises).
     static constexpr uint32_t CHAIN_TURN = 1024;
     // A launch's cycle budget counts evaluations in units of this many.
     static constexpr uint32_t RUNS_PER_CYCLE = 8;
@@ -1760,10 +1763,13 @@ class AsyncProgram {
     }
 
     // Whether the group should look for more work: too few lanes hold a
-    // promise, and (unless lanes of different operations run together) no
-    // full link waits in the stash.
-    __device__ HZ_INLINE bool lanes_wanting(uint64_t held) {
-        if (hz::wave::popc(held) >= CHAIN_MIN) return false;
+    // promise (any lane holds none, when their turn has come), and (unless
+    // lanes of different operations run together) no full link waits in the
+    // stash.
+    __device__ HZ_INLINE bool lanes_wanting(uint64_t held, bool turn) {
+        if (hz::wave::popc(held) >= CHAIN_MIN) {
+            return turn && ~held != 0ull && hz::wave::first(_grp_ctx.ready_mask) == 0u;
+        }
         return CHAIN_MIXED || hz::wave::first(_grp_ctx.ready_mask) == 0u;
     }
 
@@ -1773,7 +1779,8 @@ class AsyncProgram {
     __device__ HZ_INLINE bool chain_cycle(uint32_t pause, uint32_t left) {
         GroupContext& g = _grp_ctx;
         uint64_t held = held_lanes();
-        if (hz::wave::popc(held) < CHAIN_MIN) {
+        const bool turn = hz::wave::first(_thd_ctx.chain_streak) >= CHAIN_TURN;
+        if (hz::wave::popc(held) < CHAIN_MIN || turn) {
             held = refill(held);
             if constexpr (!CHAIN_MIXED) {
                 // Too few lanes of one operation: the stash coalesces them.
@@ -1783,21 +1790,21 @@ class AsyncProgram {
                     held = 0ull;
                 }
             }
-            if (lanes_wanting(held)) {
+            if (lanes_wanting(held, turn)) {
                 // Consulting the home queue is a device-scope load, so after
                 // a check that found nothing the group runs some cycles
                 // without one; a group that holds nothing asks every time
                 // (exec_cycle).
                 const uint32_t countdown = hz::wave::first(_thd_ctx.queue_check);
-                if (countdown != 0u) {
+                if (countdown != 0u && !turn) {
                     _thd_ctx.queue_check = countdown - 1u;
                 } else {
                     HZ_PHASE(PHASE_PULL);
-                    while (lanes_wanting(held) && queues_hint() && pull_links(1) != 0u) {
+                    while (lanes_wanting(held, turn) && queues_hint() && pull_links(1) != 0u) {
                         held = refill(held);
                         _thd_ctx.queue_pause = 0u;
                     }
-                    if (lanes_wanting(held)) {
+                    if (lanes_wanting(held, turn)) {
                         const uint32_t p = hz::wave::first(_thd_ctx.queue_pause) * 2u + 1u;
                         _thd_ctx.queue_pause = hz::wave::first(g.can_make_work) || p > QUEUE_CHECK_PERIOD - 1
                                                    ? QUEUE_CHECK_PERIOD - 1 : p;
@@ -1805,7 +1812,7 @@ class AsyncProgram {
                     }
                 }
                 HZ_PHASE(PHASE_MAKE);
-                for (uint32_t tries = 0; tries < 4 && lanes_wanting(held) && pause == 0u &&
+                for (uint32_t tries = 0; tries < 4 && lanes_wanting(held, turn) && pause == 0u &&
                                          hz::wave::first(g.can_make_work) &&
                                          hz::wave::first(_thd_ctx.make_pause) == 0u;
                      ++tries) {

@@ -733,6 +733,13 @@ int hz_pool_test(uint64_t size, const int64_t* ops, uint32_t count, uint64_t* ou
  * `report` receives a summary. */
 int hz_audit_selftest(char* report, size_t report_bytes);
 
+/* Runs, on one group, a program whose `waiting` promises (at most 63) requeue
+ * themselves until another promise has run, which the group makes after them;
+ * *passed receives how many went through. `mixed`: lanes may hold different
+ * operations. Fails if the program is not complete after `max_launches`
+ * launches of `cycles` cycles. */
+int hz_wait_selftest(uint32_t waiting, int mixed, uint32_t cycles, uint32_t max_launches, uint32_t* passed);
+
 /* Device facts used to size launches. */
 typedef struct hz_device_facts {
     int32_t device;
