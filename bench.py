@@ -14,10 +14,11 @@ and the serving load sweep (p50/p99 latency at 20-100% of peak).
 
 Consistency checks made here: the Collatz step counts of AsyncProgram,
 EventProgram and the one-thread-per-start kernel are identical (a failure
-raises: no line is printed). A further section that fails is named in the line
-("failed"), the sections after it are not run, and the exit status is 1: photon event totals and BFS levels agree between the two programs; the futures
-total and the barrier demo's count match their closed forms. The GPU tests
-check every workload, serving included, against the oracle.
+raises, and no line is printed); photon event totals and BFS levels agree
+between the two programs; the futures total and the barrier demo's count match
+their closed forms. A further section that fails is named in the line
+("failed"), the sections after it are not run, and the exit status is 1. The
+GPU tests check every workload, serving included, against the oracle.
 
     python bench.py [--gpus 1] [--steps 5] [--warmup 1] [--no-cpu] [--no-event]
                     [--no-photon] [--no-bfs] [--no-futures] [--no-barrier] [--no-serve]

@@ -180,7 +180,8 @@ struct UnitBarrier {
 
 #if defined(__HIP_DEVICE_COMPILE__)
     // Counts a fulfilment whose value is at the device's coherence point and
-    // is read there: nothing is released, nothing acquired.
+    // is read there: nothing is released, nothing acquired, so the promise
+    // that waits was written before the launch (RETURN_RELEASE = 0).
     template <typename PROGRAM>
     __device__ HZ_INLINE void count_returned(PROGRAM program) {
         if (hz::wave::atomic_add(&semaphore.sem, ~0u) == 1u && promise.disc != NO_PROMISE) program.async_call(promise);

@@ -215,7 +215,9 @@ __device__ __host__ HZ_INLINE void forward_promise(PROGRAM program, ENUM pe, Ret
 // read such values with hz_load, says so (RETURN_RELEASE = 0): a unit
 // future's value is then written through and waited for instead. (The futures
 // demo, 2^20 chains and as many joins: 2.4 million evaluations in 13.3 ms,
-// two fifths of them with a write-back; 4.7 ms without.)
+// two fifths of them with a write-back; 4.7 ms without.) The unit barriers it
+// resolves, and the promises they hold, have to be written before the launch:
+// they are read with plain loads, and nothing is acquired before that.
 template <typename PROGRAM, typename TYPE>
 __device__ __host__ HZ_INLINE void resolve_value(PROGRAM program, ReturnAdr<TYPE> adr, const TYPE& value) {
 #if defined(__HIP_DEVICE_COMPILE__)

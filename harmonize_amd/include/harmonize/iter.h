@@ -126,13 +126,13 @@ struct Share {
 //
 // On the GPU one atomic claims for the whole wavefront: per lane, what is left
 // over the launch's lanes, 1 to `most` indices (1 once fewer than `from` are
-// left). The range's counter is one
-// address for the whole device, where loads and atomics take their turn (30 ns
-// each), so a large range is claimed in large parts, and its end, or a small
-// range, one index per lane. The parts follow the counter as it is: sized
-// from a wavefront's previous claim instead, they leave too much to the last
-// few wavefronts. The lanes take the claimed indices in turn, so that a step
-// of every lane reads consecutive elements.
+// left). The range's counter is one address for the whole device, where loads
+// and atomics take their turn (30 ns each), so a large range is claimed in
+// large parts, and its end, or a small range, one index per lane. The parts
+// follow the counter as it is: sized from a wavefront's previous claim
+// instead, they leave too much to the last few wavefronts. The lanes take the
+// claimed indices in turn, so that a step of every lane reads consecutive
+// elements.
 template <typename INDEX_TYPE>
 __device__ inline void claim_share(Share<INDEX_TYPE>& share, AtomicIter<INDEX_TYPE>& range, INDEX_TYPE most,
                                    INDEX_TYPE from = 0) {

@@ -52,7 +52,14 @@ HZ_CONST_OR(GROUPS_PER_BLOCK)
 // Nonzero: a group that holds several links hands some to groups that have
 // none (for work that grows from few seeds). Not a reference constant.
 HZ_CONST_OR(SHARE_WORK)
+// Zero: a group that takes a queued link acquires nothing besides it. For
+// promises that carry all they need, or read the rest with hz_load. Default 1.
+// Not a reference constant.
 HZ_CONST_OR(LINK_ACQUIRE)
+// Zero: resolving a unit future publishes the returned value only, and reads
+// the future's barrier and its promise with plain loads. For value-returning
+// operations that hand over nothing else, values read with hz_load, and
+// barriers built before the launch. Default 1. Not a reference constant.
 HZ_CONST_OR(RETURN_RELEASE)
 // Nonzero: a group runs its ready links oldest first (the order in which
 // they filled), rather than by stash position. Work whose later promises can

@@ -79,10 +79,6 @@ __device__ HZ_INLINE void atomic_store(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <typename T>
-__device__ HZ_INLINE void atomic_store_release(T* p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
 __device__ HZ_INLINE T atomic_or(T* p, T v) {
     return __hip_atomic_fetch_or(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -28,8 +28,8 @@ struct BarrierDemoState {
     RemappingBarrier<OpUnion<BarrierStep>>* barrier;
 };
 
-// What a thread has claimed and not started, and the evaluations it has yet
-// to add to the counter.
+// The id a thread has claimed (make_work starts it at once, so none is left
+// when a launch ends), and the evaluations it has yet to add to the counter.
 struct BarrierDemoThread {
     util::iter::Share<unsigned int> ids;
     unsigned int steps;
@@ -84,8 +84,6 @@ struct BarrierDemoSpec {
 
     template <typename PROGRAM>
     __device__ static void finalize(PROGRAM prog) {
-        unsigned int id;
-        while (prog.thread.ids.step(id)) prog.template sync<BarrierStep>(id);
         unsigned int steps = prog.thread.steps;
 #if defined(__HIP_DEVICE_COMPILE__)
         for (int d = 32; d >= 1; d >>= 1) steps += __shfl_xor(steps, d, 64);

@@ -171,13 +171,8 @@ namespace resident {
 // waits until its earlier stores have completed (s_waitcnt), so whoever sees
 // the publishing store sees them too. Acquire and release orderings would add
 // an L2 invalidate or write-back to every claim and poll; none of the shared
-// data needs them. The signal fences keep the compiler from moving memory
-// operations across the wait.
-__device__ HZ_INLINE void stores_done() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
+// data needs them.
+using hz::wave::stores_done;
 
 template <typename T>
 __device__ HZ_INLINE T ld(const T* p) {
@@ -822,10 +817,10 @@ struct ResidentPhotonKind {
     static const size_t STASH_SIZE = HZ_PHOTON_STASH;
     static const size_t CHAIN_PASSES = 1;
 
-    // Eight photons per lane while BULK_FROM or more are left, else one. Bulk claims also take the job's tally into LDS. (One
-    // share of what is left per lane, as for Collatz, lowers the photon
-    // serving peak by a quarter; four per lane, the photon program's own
-    // claim, by 6%.)
+    // Eight photons per lane while BULK_FROM or more are left, else one. Bulk
+    // claims also take the job's tally into LDS. (One share of what is left
+    // per lane, as for Collatz, lowers the photon serving peak by a quarter;
+    // four per lane, the photon program's own claim, by 6%.)
     static constexpr unsigned int BULK_FROM = 1u << 17;
     __device__ static HZ_INLINE unsigned int per_lane(unsigned int left, unsigned int) {
         return left >= BULK_FROM ? 8u : 1u;
