@@ -228,8 +228,11 @@ class EventProgram {
         : _dev_ctx(d_c), _grp_ctx(g_c), _thd_ctx(t_c), device(d), group(g), thread(t) {}
 
    protected:
+    // (A choice, not an index: indexed by a variable, the context is kept in
+    // LDS, a copy per lane.)
     __device__ unsigned int* queue_row(unsigned int which, OpDisc op, unsigned int word) {
-        return _dev_ctx.queues[which] + ((size_t)op * WORDS + word) * _dev_ctx.capacity;
+        unsigned int* queue = which != 0u ? _dev_ctx.queues[1] : _dev_ctx.queues[0];
+        return queue + ((size_t)op * WORDS + word) * _dev_ctx.capacity;
     }
 
     __device__ Segment& segment(OpDisc op, uint32_t s) { return _dev_ctx.status->seg[op][s]; }

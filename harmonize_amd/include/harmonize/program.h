@@ -8,8 +8,26 @@
 #include "async.h"
 #include "event.h"
 
-template <typename ProgType>
+namespace hz {
+template <typename P>
+struct IsAsync : std::false_type {};
+template <typename S>
+struct IsAsync<AsyncProgram<S>> : std::true_type {};
+}  // namespace hz
+
+template <typename ProgType, typename std::enable_if<hz::IsAsync<ProgType>::value, int>::type = 0>
 __global__ void __launch_bounds__(ProgType::WORK_GROUP_SIZE)
+    _hz_exec_kernel(typename ProgType::DeviceContext ctx, typename ProgType::DeviceState state, unsigned int n) {
+    ProgType::kernel_exec(ctx, state, n);
+}
+
+// A generation's groups are as many as the device holds at eight wavefronts a
+// SIMD, which takes at most 80 scalar registers (the device adds its own, so
+// with 92 of them seven are resident, while the occupancy query says eight): a
+// last round of a few groups cost large generations a third of their time
+// (2^26 Collatz starts 234 ms with 92, 184 with 80).
+template <typename ProgType, typename std::enable_if<!hz::IsAsync<ProgType>::value, int>::type = 0>
+__global__ void __launch_bounds__(ProgType::WORK_GROUP_SIZE) __attribute__((amdgpu_num_sgpr(80)))
     _hz_exec_kernel(typename ProgType::DeviceContext ctx, typename ProgType::DeviceState state, unsigned int n) {
     ProgType::kernel_exec(ctx, state, n);
 }
@@ -46,13 +64,6 @@ void AsyncProgram<PROGRAM_SPEC>::Instance::reset(hipStream_t stream) {
                        stream, to_context());
     util::host::auto_throw(hipGetLastError());
 }
-
-namespace hz {
-template <typename P>
-struct IsAsync : std::false_type {};
-template <typename S>
-struct IsAsync<AsyncProgram<S>> : std::true_type {};
-}  // namespace hz
 
 // Prepares an instance for execution. For an AsyncProgram this empties its
 // queues and clears its status (reference AsyncProgram::init_program,
