@@ -58,10 +58,10 @@ int resident_groups_of() {
     static std::atomic<int> known[64];
     int dev = 0;
     check(hipGetDevice(&dev), "hipGetDevice");
-    if (dev < 0 || dev >= 64) return resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
+    if (dev < 0 || dev >= 64) return resident_groups(hz::exec_kernel<P>(), (int)P::WORK_GROUP_SIZE);
     int n = known[dev].load(std::memory_order_relaxed);
     if (n == 0) {
-        n = resident_groups(_hz_exec_kernel<P>, (int)P::WORK_GROUP_SIZE);
+        n = resident_groups(hz::exec_kernel<P>(), (int)P::WORK_GROUP_SIZE);
         known[dev].store(n, std::memory_order_relaxed);
     }
     return n;

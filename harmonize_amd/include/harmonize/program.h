@@ -15,7 +15,7 @@ template <typename S>
 struct IsAsync<AsyncProgram<S>> : std::true_type {};
 }  // namespace hz
 
-template <typename ProgType, typename std::enable_if<hz::IsAsync<ProgType>::value, int>::type = 0>
+template <typename ProgType>
 __global__ void __launch_bounds__(ProgType::WORK_GROUP_SIZE)
     _hz_exec_kernel(typename ProgType::DeviceContext ctx, typename ProgType::DeviceState state, unsigned int n) {
     ProgType::kernel_exec(ctx, state, n);
@@ -26,11 +26,23 @@ __global__ void __launch_bounds__(ProgType::WORK_GROUP_SIZE)
 // with 92 of them seven are resident, while the occupancy query says eight): a
 // last round of a few groups cost large generations a third of their time
 // (2^26 Collatz starts 234 ms with 92, 184 with 80).
-template <typename ProgType, typename std::enable_if<!hz::IsAsync<ProgType>::value, int>::type = 0>
+template <typename ProgType>
 __global__ void __launch_bounds__(ProgType::WORK_GROUP_SIZE) __attribute__((amdgpu_num_sgpr(80)))
-    _hz_exec_kernel(typename ProgType::DeviceContext ctx, typename ProgType::DeviceState state, unsigned int n) {
+    _hz_generation_kernel(typename ProgType::DeviceContext ctx, typename ProgType::DeviceState state, unsigned int n) {
     ProgType::kernel_exec(ctx, state, n);
 }
+
+namespace hz {
+// The kernel of a program type's launches.
+template <typename P>
+constexpr auto exec_kernel() {
+    if constexpr (IsAsync<P>::value) {
+        return &_hz_exec_kernel<P>;
+    } else {
+        return &_hz_generation_kernel<P>;
+    }
+}
+}  // namespace hz
 
 template <typename ProgType>
 __global__ void __launch_bounds__(256) _hz_async_reset_kernel(typename ProgType::DeviceContext ctx) {
@@ -89,7 +101,7 @@ template <typename ProgType>
 __host__ void exec(typename ProgType::Instance& instance, size_t group_count, size_t n, hipStream_t stream = nullptr) {
     if (group_count == 0) group_count = 1;
     auto ctx = instance.to_context();
-    hipLaunchKernelGGL(_hz_exec_kernel<ProgType>, dim3((unsigned)blocks_for<ProgType>(group_count)),
+    hipLaunchKernelGGL(hz::exec_kernel<ProgType>(), dim3((unsigned)blocks_for<ProgType>(group_count)),
                        dim3((unsigned)ProgType::WORK_GROUP_SIZE), 0, stream, ctx, instance.device_state,
                        (unsigned int)(n > 0xFFFFFFFFull ? 0xFFFFFFFFull : n));
     if constexpr (!hz::IsAsync<ProgType>::value) {
