@@ -323,8 +323,10 @@ extern "C" int hz_resident_create(const hz_resident_config* config, hz_resident*
         if (c.policy > R::SMALLEST_FIRST) throw std::invalid_argument("hz_resident_create: unknown policy");
         if (c.kind == HZ_JOB_PHOTON && c.policy == R::SMALLEST_FIRST) {
             // A photon server claiming smallest job first once stopped making
-            // progress in a serving sweep, for a reason not yet found; the
-            // combination stays refused until it is.
+            // progress in a serving sweep. Completion words that two jobs in
+            // flight could share (claim_word.h) explain it; the sweep has not
+            // been run on a device since they are apart, so the combination
+            // stays refused.
             throw std::invalid_argument("hz_resident_create: photon jobs are claimed in arrival order only");
         }
         if (c.kind != HZ_JOB_COLLATZ && c.kind != HZ_JOB_PHOTON) {

@@ -211,7 +211,7 @@ __device__ inline void bfs_relax_wave(PROGRAM& prog, unsigned int job, const Bfs
             // no look at its level. The hints of a graph take an eighth of
             // its levels' bytes, so more of them are found in the XCD's L2:
             // 57 % of all requests, where it was a third (fetched beyond the
-            // L2 58 to 34 GB).
+            // L2: 58 GB before, 27 to 30 GB now).
 #pragma unroll
             for (int k = 0; k < CH; ++k) {
                 at[k] = row[edges.owner[k]].vertex + (unsigned int)edges.w[k];
