@@ -325,6 +325,10 @@ typedef struct hz_run_config {
  * evaluated, queued or held by a barrier. A violation fails the run with
  * HZ_ERR_RUNTIME naming it. */
 #define HZ_RUN_AUDIT 2u
+/* A BFS batch's search looks levels up through level hints (four bits per
+ * vertex) whatever the batch's size; by default only where that is faster.
+ * Levels are the same either way. */
+#define HZ_RUN_LEVEL_HINTS 4u
 
 typedef struct hz_run_stats {
     uint64_t promises;        /* promises evaluated */
